@@ -166,28 +166,93 @@ __device__ __forceinline__ void block_sum4(double* v)
     __syncthreads();
 }
 
-// Block-wide lexicographic maximum of every thread's 4-vector, the same way.
-__device__ __forceinline__ void block_lexmax4(double* v)
+// Maximum over the wavefront of one double per lane, none of them NaN, to
+// every lane (an exact selection, so the order of combination gives the same
+// bits): a DPP scan within each row of 16 lanes, then across the rows, which
+// leaves the maximum in lane 63.  Lanes the shifted source does not reach
+// take -1, a lower bound of every caller's values.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double dpp_shift(double v)
 {
-    __shared__ double wres[kBlock / 64][4];
-    for (int o = 32; o > 0; o >>= 1) {
-        double c[4];
+    constexpr int kNeg1Hi = (int)0xbff00000;  // -1.0 = 0xbff00000'00000000
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(kNeg1Hi, __double2hiint(v), CTRL, ROW_MASK, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double wave_max(double v)
+{
+    v = fmax(v, dpp_shift<0x111, 0xf>(v));  // row_shr:1
+    v = fmax(v, dpp_shift<0x112, 0xf>(v));  // row_shr:2
+    v = fmax(v, dpp_shift<0x114, 0xf>(v));  // row_shr:4
+    v = fmax(v, dpp_shift<0x118, 0xf>(v));  // row_shr:8
+    v = fmax(v, dpp_shift<0x142, 0xa>(v));  // row_bcast:15, rows 1 and 3
+    v = fmax(v, dpp_shift<0x143, 0xc>(v));  // row_bcast:31, rows 2 and 3
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                            __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// Lane l's value of v, to every lane (l uniform).
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// Lexicographic maximum over the wavefront of every lane's 4-vector (entries
+// >= -1 or NaN, NaN above every number), to every lane: the lanes that hold
+// the largest first component, among them those with the largest second, and
+// so on until one is left (usually at once); the survivors' vectors are
+// equal.  Every lane must be active.
+__device__ __forceinline__ void wave_lexmax4(double* v)
+{
+    uint64_t in = ~(uint64_t)0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) c[q] = __shfl_xor(v[q], o);
-        if (lex_less(v, c))
-#pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = c[q];
+    for (int q = 0; q < 4; ++q) {
+        const bool mine = (in >> (threadIdx.x & 63)) & 1;
+        const uint64_t nan = __ballot(mine && isnan(v[q]));
+        if (nan)
+            in = nan;
+        else {
+            const double m = wave_max(mine ? v[q] : -1.0);
+            in = __ballot(mine && v[q] == m);
+        }
+        if (!(in & (in - 1))) break;
     }
+    const int l = (int)__ffsll((unsigned long long)in) - 1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = lane_value(v[q], l);
+}
+
+// One 4-vector per wavefront into LDS, and (after a barrier) their
+// lexicographic maximum, to every lane.
+__device__ __forceinline__ void store_wave4(const double* v, double (*wres)[4])
+{
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
         for (int q = 0; q < 4; ++q) wres[threadIdx.x >> 6][q] = v[q];
+}
+
+__device__ __forceinline__ void lexmax4_of_waves(double* v, const double (*wres)[4])
+{
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = l < kBlock / 64 ? wres[l & (kBlock / 64 - 1)][q] : -1.0;
+    wave_lexmax4(v);
+}
+
+// Block-wide lexicographic maximum of every thread's 4-vector (entries >= -1
+// or NaN): each wavefront's by DPP and ballots, then the four wavefronts'.
+// Every thread gets the result.  A butterfly of shuffles over whole vectors
+// with a branching comparison per step took 4.0 us of every stencil kernel
+// with the residual viscosity, whatever its size.
+__device__ __forceinline__ void block_lexmax4(double* v)
+{
+    __shared__ double wres[kBlock / 64][4];
+    wave_lexmax4(v);
+    store_wave4(v, wres);
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = wres[0][q];
-    for (int w = 1; w < kBlock / 64; ++w)
-        if (lex_less(v, wres[w]))
-#pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = wres[w][q];
+    lexmax4_of_waves(v, wres);
     __syncthreads();
 }
 

@@ -356,10 +356,11 @@ constexpr int kSeqViscosity = 1, kSeqTominec = 2, kSeqFlyer = 3;
 // for the transposed pass du_i -= gamma sum_r lap_ri L_r (hyperviscosity.jl:
 // 111-134, the factors of H = lap' lap).
 // Residual-viscosity norms in the stencil kernels: thread b loads the max
-// pass's partial b at kernel start (at most kBlock partials) and keeps it
-// in registers untouched, so the load overlaps the halo staging and the
-// stencil loop instead of holding them up; the block reduces the partials
-// just before the viscosity is needed.  Every block gets the same bits.
+// pass's partial b at kernel start (at most kBlock partials).  With LDS tiles
+// each wavefront reduces its partials to one vector before the barrier of the
+// halo staging, while the halo's loads are in flight, and the four vectors
+// are combined where the viscosity is needed; without tiles the block reduces
+// them there.  Every block gets the same bits.
 __device__ __forceinline__ void prefetch_max_partials(const RhsArgs& a, double* pm)
 {
     if ((int)threadIdx.x < a.nparts)
@@ -367,9 +368,13 @@ __device__ __forceinline__ void prefetch_max_partials(const RhsArgs& a, double* 
         for (int v = 0; v < 4; ++v) pm[v] = a.pmax[4 * threadIdx.x + v];
 }
 
-__device__ __forceinline__ void finish_norms(const RhsArgs& a, double* pm, double* ninf)
+template <bool TL>
+__device__ __forceinline__ void finish_norms(const RhsArgs& a, double* pm, const double (*wmax)[4], double* ninf)
 {
-    block_lexmax4(pm);
+    if constexpr (TL)
+        lexmax4_of_waves(pm, wmax);
+    else
+        block_lexmax4(pm);
 #pragma unroll
     for (int v = 0; v < 4; ++v) ninf[v] = (pm[v] == 0.0) ? DBL_EPSILON : pm[v];
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.norms_out)
@@ -468,11 +473,13 @@ __device__ __forceinline__ void flux_nb(const EqParams& e, const double* r, doub
 // Node of this thread and, with LDS tiles (TL), the tile's stencil halo
 // staged in lds: halo entry q holds the record of node ha_ids[ha_off[t] + q].
 // Returns -1 for threads without a node (after the block barrier) and
-// kNoBlock when the whole block has none.
+// kNoBlock when the whole block has none.  rvres: reduce each wavefront's
+// partials pm into wmax on the way (see prefetch_max_partials).
 constexpr int64_t kNoBlock = -2;
 
 template <int V, bool TL>
-__device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds)
+__device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds, bool rvres, double* pm,
+                                                double (*wmax)[4])
 {
     if constexpr (TL) {
         const int64_t t = remapped_block();
@@ -491,6 +498,10 @@ __device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds)
             } else {
                 store_state<V>(lds, q, r);
             }
+        }
+        if (rvres) {
+            wave_lexmax4(pm);
+            store_wave4(pm, wmax);
         }
         __syncthreads();
         const int64_t i = t * kBlock + threadIdx.x;
@@ -515,7 +526,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds);
+    __shared__ double wmax[kBlock / 64][4];
+    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
     if (i_node == kNoBlock) return;  // whole block
     // a thread without a node shadows the last node until the block-wide
     // norm reduction, then leaves
@@ -594,7 +606,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
             load_state<V>(a.u, i, ui);
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
-            if (rvres) finish_norms(a, pm, ninf);
+            if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, i, ui, du, ninf, &code);
             a.eps[i] = e;
@@ -689,7 +701,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds);
+    __shared__ double wmax[kBlock / 64][4];
+    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
     if (i_node == kNoBlock) return;  // whole block
     // a thread without a node shadows the last node until the block-wide
     // norm reduction, then leaves
@@ -711,7 +724,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
             load_state<V>(a.u, i, ui);
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
-            if (rvres) finish_norms(a, pm, ninf);
+            if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, i, ui, du, ninf, &code);
             a.eps[i] = e;
@@ -752,7 +765,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds);
+    __shared__ double wmax[kBlock / 64][4];
+    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
     if (i_node == kNoBlock) return;  // whole block
     // a thread without a node shadows the last node until the block-wide
     // norm reduction, then leaves
@@ -846,7 +860,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
         if constexpr (RV) {
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
-            if (rvres) finish_norms(a, pm, ninf);
+            if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, i, ui, du, ninf, &code);
             a.eps[i] = e;

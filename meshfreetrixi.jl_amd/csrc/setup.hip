@@ -627,40 +627,6 @@ struct WeightsArgs {
     int* status;
 };
 
-// Maximum over the wavefront of one double per lane (an exact selection,
-// so any combination order gives the same bits), returned to every lane:
-// a DPP max-scan within each row of 16 lanes (row_shr 1, 2, 4, 8), then
-// across rows (row_bcast 15, 31), which leaves the maximum in lane 63.
-// Lanes the shifted source does not reach take -1, below every |x|; every
-// lane of the wavefront must be active.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double dpp_shift(double v)
-{
-    constexpr int kNeg1Hi = (int)0xbff00000;  // -1.0 = 0xbff00000'00000000
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROW_MASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(kNeg1Hi, __double2hiint(v), CTRL, ROW_MASK, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double wave_max(double v)
-{
-    v = fmax(v, dpp_shift<0x111, 0xf>(v));  // row_shr:1
-    v = fmax(v, dpp_shift<0x112, 0xf>(v));  // row_shr:2
-    v = fmax(v, dpp_shift<0x114, 0xf>(v));  // row_shr:4
-    v = fmax(v, dpp_shift<0x118, 0xf>(v));  // row_shr:8
-    v = fmax(v, dpp_shift<0x142, 0xa>(v));  // row_bcast:15, rows 1 and 3
-    v = fmax(v, dpp_shift<0x143, 0xc>(v));  // row_bcast:31, rows 2 and 3
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
-                            __builtin_amdgcn_readlane(__double2loint(v), 63));
-}
-
-// Lane l's value of v, to every lane (l uniform).
-__device__ __forceinline__ double lane_value(double v, int l)
-{
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
-                            __builtin_amdgcn_readlane(__double2loint(v), l));
-}
-
 // Interchange of rows p and q of B held one row per lane (p, q uniform).
 __device__ __forceinline__ void lanes_swap(double& b0, double& b1, int lane, int p, int q)
 {
