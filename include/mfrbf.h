@@ -355,8 +355,11 @@ int mf_ssprk33_vjp(mf_ctx* ctx, double t0, double dt, int n_steps, int checkpoin
                    double* loss);
 
 /* ------------------------------------------------------------- tuning */
-#define MF_TUNE_FLUX_BATCH 0      /* stencil entries loaded per batch: 3, 5, 6, 10 (0 = default) */
-#define MF_TUNE_TRANSPOSE_BATCH 1 /* transposed entries loaded per batch: 2, 4, 8 (0 = default) */
+#define MF_TUNE_FLUX_BATCH 0      /* stencil entries in flight per thread: 3, 5 (one batch at a time), 6,
+                                     10 (two batches of 3, 5 in turn); 0 (default): by the number of
+                                     LDS tiles per compute unit */
+#define MF_TUNE_TRANSPOSE_BATCH 1 /* transposed entries per batch, two batches in turn: 2, 4, 8; 0
+                                     (default): by the number of LDS tiles per compute unit */
 #define MF_TUNE_NODE_ORDER 2      /* internal node order for the next mf_set_points: 0 Morton
                                      (default), 1 the caller's order; precision is ignored */
 #define MF_TUNE_TILES 3           /* 1 (default): stage stencil halos in LDS where they fit;

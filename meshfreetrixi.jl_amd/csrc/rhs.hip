@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <type_traits>
 
 #include "mf_device.h"
 
@@ -307,9 +308,9 @@ __device__ __forceinline__ void emit_staged(const RhsArgs& a, int64_t i, const d
 
 // Residual/upwind viscosity at node i (hyperviscosity.jl:246-349): eps_uw
 // from the local state, eps_rv from |approx_du - du| scaled by the global
-// norms, then the choice of update_visc!.
-__device__ __forceinline__ double node_viscosity(const RhsArgs& a, int64_t i, const double* ui,
-                                                 const double* dui, const double* ninf, int8_t* code)
+// norms, then the choice of update_visc!.  ad: approx_du at the node.
+__device__ __forceinline__ double node_viscosity(const RhsArgs& a, const double* ui, const double* dui,
+                                                 const double* ad, const double* ninf, int8_t* code)
 {
     const double gam = a.eq.gamma;
     const double rho = ui[0], m1 = ui[1], m2 = ui[2], E = ui[3];
@@ -323,8 +324,6 @@ __device__ __forceinline__ double node_viscosity(const RhsArgs& a, int64_t i, co
         *code = 1;
         return eps_uw;
     }
-    double ad[4];
-    load_state<4>(a.approx, i, ad);
     double mr = 0.0;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -470,20 +469,15 @@ __device__ __forceinline__ void flux_nb(const EqParams& e, const double* r, doub
         flux_xy<V>(e, r, f1, f2);
 }
 
-// Node of this thread and, with LDS tiles (TL), the tile's stencil halo
-// staged in lds: halo entry q holds the record of node ha_ids[ha_off[t] + q].
-// Returns -1 for threads without a node (after the block barrier) and
-// kNoBlock when the whole block has none.  rvres: reduce each wavefront's
-// partials pm into wmax on the way (see prefetch_max_partials).
-constexpr int64_t kNoBlock = -2;
-
+// With LDS tiles (TL), stages the stencil halo of tile t in lds: halo entry q
+// holds the record of node ha_ids[ha_off[t] + q]; ends with a block barrier.
+// rvres: reduce each wavefront's partials pm into wmax on the way (see
+// prefetch_max_partials).
 template <int V, bool TL>
-__device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds, bool rvres, double* pm,
-                                                double (*wmax)[4])
+__device__ __forceinline__ void stage_halo_a(const RhsArgs& a, int64_t t, double* lds, bool rvres, double* pm,
+                                             double (*wmax)[4])
 {
     if constexpr (TL) {
-        const int64_t t = remapped_block();
-        if (t >= a.n_tiles) return kNoBlock;  // whole block
         const int64_t h0 = a.ha_off[t];
         const int nh = (int)(a.ha_off[t + 1] - h0);
         for (int q = threadIdx.x; q < nh; q += kBlock) {
@@ -504,12 +498,61 @@ __device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds, b
             store_wave4(pm, wmax);
         }
         __syncthreads();
-        const int64_t i = t * kBlock + threadIdx.x;
-        return i < a.N ? i : -1;
+    }
+}
+
+// base[lane] with a uniform base: a scalar base address and a 32-bit lane
+// offset, instead of a 64-bit address per entry and lane.
+template <class T>
+__device__ __forceinline__ T at_lane(const T* base, uint32_t lane)
+{
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + lane * (uint32_t)sizeof(T));
+}
+
+// Entry s of this thread's node: tile-major (TL; tile blk, padded with zeros
+// past the last node) or slot-major.
+template <bool TL, class T>
+__device__ __forceinline__ T entry_of(const T* p, int64_t blk, int K, int s, int64_t N, int64_t i)
+{
+    if constexpr (TL)
+        return at_lane(p + (blk * K + s) * kBlock, threadIdx.x);
+    else
+        return p[(int64_t)s * N + i];
+}
+
+// One batch of stencil entries of a row: halo positions or nodes, (Dx, Dy)
+// (or one of them), Flyer and Laplacian weights.
+template <class W, class W1, int BT>
+struct FluxBatch {
+    int32_t j[BT];
+    W w[BT];
+    W1 hw[BT], lw[BT];
+};
+
+// The K entries of a row in batches of BT.  PF: the loads of the next batch
+// are issued before the batch at hand is used, from two sets of registers in
+// turn, and the caller issues the first batch's (q0) before it stages the
+// halo.  sched_barrier: the scheduler otherwise sinks each load to its use.
+template <int BT, bool PF, class Q, class Load, class Use>
+__device__ __forceinline__ void for_batches(int K, Q& q0, Load load, Use use)
+{
+    if constexpr (PF) {
+        Q q1;
+#pragma unroll 1
+        for (int s0 = 0; s0 < K; s0 += 2 * BT) {
+            if (s0 + BT < K) load(s0 + BT, q1);
+            __builtin_amdgcn_sched_barrier(0);
+            use(q0);
+            if (s0 + 2 * BT < K) load(s0 + 2 * BT, q0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s0 + BT < K) use(q1);
+        }
     } else {
-        if (remapped_block() * kBlock >= a.N) return kNoBlock;  // whole block
-        const int64_t i = remapped_node();
-        return i < a.N ? i : -1;
+#pragma unroll 1
+        for (int s0 = 0; s0 < K; s0 += BT) {
+            load(s0, q0);
+            use(q0);
+        }
     }
 }
 
@@ -518,79 +561,86 @@ __device__ __forceinline__ int64_t stage_halo_a(const RhsArgs& a, double* lds, b
 // so BT gathers are in flight per thread.  Entries past K read a valid node
 // with weight 0.  TL: neighbour records come from the LDS halo, addressed
 // by 16-bit halo positions (same slot-major layout as idx).
-template <int V, int NS, int HVK, bool RV, int BT, bool TL>
+template <int V, int NS, int HVK, bool RV, int BT, bool PF, bool TL>
 __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    const int64_t blk = remapped_block();
+    if (blk * kBlock >= a.N) return;  // whole block
+    const int64_t N = a.N;
+    const int K = NS ? NS : a.k;
+    const int64_t i_node = blk * kBlock + threadIdx.x;
+    // a thread without a node shadows the last node until the block-wide
+    // norm reduction, then leaves
+    const bool live = i_node < N;
+    const int64_t i = live ? i_node : N - 1;
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
-    __shared__ double wmax[kBlock / 64][4];
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
-    if (i_node == kNoBlock) return;  // whole block
-    // a thread without a node shadows the last node until the block-wide
-    // norm reduction, then leaves
-    const bool live = i_node >= 0;
-    if (!rvres && !live) return;
-    const int64_t i = live ? i_node : a.N - 1;
-    const int64_t N = a.N;
-    const int K = NS ? NS : a.k;
-    double ax[V], ay[V], gx[V], gy[V], hh[V], ll[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) ax[v] = ay[v] = gx[v] = gy[v] = hh[v] = ll[v] = 0.0;
-#pragma unroll 1
-    for (int s0 = 0; s0 < K; s0 += BT) {
-        int32_t j[BT];
-        double2 w[BT];
-        double hw[BT], lw[BT];
+    auto load = [&](int s0, FluxBatch<double2, double, BT>& q) {
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             const int s = s0 + b;
             if ((NS && NS % BT == 0) || s < K) {
-                const int64_t q = TL ? tm_pos(s, i, K) : (int64_t)s * N + i;
                 if constexpr (TL)
-                    j[b] = a.la[q];
+                    q.j[b] = entry_of<TL>(a.la, blk, K, s, N, i);
                 else
-                    j[b] = a.idx[q];
-                w[b] = a.wxy[q];
-                if constexpr (FLY) hw[b] = a.hv[q];
-                if constexpr (TOM) lw[b] = a.lap[q];
+                    q.j[b] = entry_of<TL>(a.idx, blk, K, s, N, i);
+                q.w[b] = entry_of<TL>(a.wxy, blk, K, s, N, i);
+                if constexpr (FLY) q.hw[b] = entry_of<TL>(a.hv, blk, K, s, N, i);
+                if constexpr (TOM) q.lw[b] = entry_of<TL>(a.lap, blk, K, s, N, i);
             } else {
-                j[b] = TL ? 0 : (int32_t)i;
-                w[b] = make_double2(0.0, 0.0);
-                hw[b] = lw[b] = 0.0;
+                q.j[b] = TL ? 0 : (int32_t)i;
+                q.w[b] = make_double2(0.0, 0.0);
+                q.hw[b] = q.lw[b] = 0.0;
             }
         }
+    };
+    FluxBatch<double2, double, BT> q0;
+    if constexpr (PF) load(0, q0);
+    __shared__ double wmax[kBlock / 64][4];
+    stage_halo_a<V, TL>(a, blk, lds, rvres, pm, wmax);
+    if (!rvres && !live) return;
+    double ui[V], ad[V];  // the node's state and approx_du, in flight through the loop
+    if constexpr (RV) {
+        load_state<V>(a.u, i, ui);
+        if (rvres) load_state<V>(a.approx, i, ad);
+    }
+    double ax[V], ay[V], gx[V], gy[V], hh[V], ll[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) ax[v] = ay[v] = gx[v] = gy[v] = hh[v] = ll[v] = 0.0;
+    auto use = [&](const FluxBatch<double2, double, BT>& q) {
         double uj[BT][TL ? rec_len<V>() : V];
 #pragma unroll
-        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, j[b], uj[b]);
+        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, q.j[b], uj[b]);
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             double f1[V], f2[V];
             flux_nb<V, TL>(a.eq, uj[b], f1, f2);
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                ax[v] = fma(w[b].x, f1[v], ax[v]);
-                ay[v] = fma(w[b].y, f2[v], ay[v]);
+                ax[v] = fma(q.w[b].x, f1[v], ax[v]);
+                ay[v] = fma(q.w[b].y, f2[v], ay[v]);
             }
             if constexpr (RV) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    gx[v] = fma(w[b].x, uj[b][v], gx[v]);
-                    gy[v] = fma(w[b].y, uj[b][v], gy[v]);
+                    gx[v] = fma(q.w[b].x, uj[b][v], gx[v]);
+                    gy[v] = fma(q.w[b].y, uj[b][v], gy[v]);
                 }
             }
             if constexpr (FLY) {
 #pragma unroll
-                for (int v = 0; v < V; ++v) hh[v] = fma(hw[b], uj[b][v], hh[v]);
+                for (int v = 0; v < V; ++v) hh[v] = fma(q.hw[b], uj[b][v], hh[v]);
             }
             if constexpr (TOM) {
 #pragma unroll
-                for (int v = 0; v < V; ++v) ll[v] = fma(lw[b], uj[b][v], ll[v]);
+                for (int v = 0; v < V; ++v) ll[v] = fma(q.lw[b], uj[b][v], ll[v]);
             }
         }
-    }
+    };
+    for_batches<BT, PF>(K, q0, load, use);
     double du[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) du[v] = -ax[v] - ay[v];
@@ -602,13 +652,11 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
     }
     if constexpr (RV || TOM) {
         if constexpr (RV) {
-            double ui[V];
-            load_state<V>(a.u, i, ui);
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
-            const double e = node_viscosity(a, i, ui, du, ninf, &code);
+            const double e = node_viscosity(a, ui, du, ad, ninf, &code);
             a.eps[i] = e;
             a.epsc[i] = code;
             double g[2 * V];
@@ -646,87 +694,121 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
 // first, then the adds in entry order).  PASS 0: x flux (and D_x u),
 // 1: y flux (and D_y u), 2: Flyer term, 3: L = lap u of the Tominec source
 // (lap * u in CSC order, as the first factor of its H = lap' lap).
-template <int V, int NS, bool RV, int BT, int PASS, bool TL>
-__device__ __forceinline__ void ref_pass(const RhsArgs& a, int64_t i, int K, double* du, double* g,
-                                         const double* lds)
+template <int V, int NS, int BT, bool TL>
+__device__ __forceinline__ void ref_load(const RhsArgs& a, int64_t blk, int64_t i, int K, const double* __restrict__ wsrc, int s0,
+                                         FluxBatch<double, double, BT>& q)
 {
-    const int64_t N = a.N;
-    const double* __restrict__ wsrc = PASS == 0 ? a.wx_s : (PASS == 1 ? a.wy_s : (PASS == 2 ? a.hv_s : a.lap_s));
-    const double ng = -a.hv_gamma;
-#pragma unroll 1
-    for (int s0 = 0; s0 < K; s0 += BT) {
-        int32_t j[BT];
-        double w[BT];
 #pragma unroll
-        for (int b = 0; b < BT; ++b) {
-            const int s = s0 + b;
-            const bool in = (NS && NS % BT == 0) || s < K;
-            const int64_t q = TL ? tm_pos(in ? s : s0, i, K) : (int64_t)(in ? s : s0) * N + i;
-            if constexpr (TL)
-                j[b] = a.la_s[q];
-            else
-                j[b] = a.idx_s[q];
-            w[b] = wsrc[q];
-        }
+    for (int b = 0; b < BT; ++b) {
+        const int s = s0 + b;
+        const bool in = (NS && NS % BT == 0) || s < K;
+        if constexpr (TL)
+            q.j[b] = entry_of<TL>(a.la_s, blk, K, in ? s : s0, a.N, i);
+        else
+            q.j[b] = entry_of<TL>(a.idx_s, blk, K, in ? s : s0, a.N, i);
+        q.w[b] = entry_of<TL>(wsrc, blk, K, in ? s : s0, a.N, i);
+    }
+}
+
+// wnext: the weights whose first batch is loaded into q0 during the last
+// batches of this pass (null: none).
+template <int V, int NS, bool RV, int BT, bool PF, int PASS, bool TL>
+__device__ __forceinline__ void ref_pass(const RhsArgs& a, int64_t blk, int64_t i, int K, double* du, double* g, const double* lds,
+                                         const double* __restrict__ wsrc, FluxBatch<double, double, BT>& q0,
+                                         const double* __restrict__ wnext)
+{
+    const double ng = -a.hv_gamma;
+    auto use = [&](int s0, const FluxBatch<double, double, BT>& q) {
         double uj[BT][TL ? rec_len<V>() : V];
 #pragma unroll
-        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, j[b], uj[b]);
+        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, q.j[b], uj[b]);
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             if (!((NS && NS % BT == 0) || s0 + b < K)) continue;
+            const double w = q.w[b];
             if constexpr (PASS == 2) {
 #pragma unroll
-                for (int v = 0; v < V; ++v) du[v] = du[v] + w[b] * (uj[b][v] * ng);
+                for (int v = 0; v < V; ++v) du[v] = du[v] + w * (uj[b][v] * ng);
             } else if constexpr (PASS == 3) {
 #pragma unroll
-                for (int v = 0; v < V; ++v) du[v] = du[v] + w[b] * uj[b][v];
+                for (int v = 0; v < V; ++v) du[v] = du[v] + w * uj[b][v];
             } else {
                 double f1[V], f2[V];
                 flux_nb<V, TL>(a.eq, uj[b], f1, f2);
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    du[v] = du[v] - w[b] * (PASS == 0 ? f1[v] : f2[v]);
-                    if constexpr (RV) g[v] = g[v] + w[b] * uj[b][v];
+                    du[v] = du[v] - w * (PASS == 0 ? f1[v] : f2[v]);
+                    if constexpr (RV) g[v] = g[v] + w * uj[b][v];
                 }
             }
         }
+    };
+    // as for_batches, with PF chained to the next pass
+    if constexpr (!PF) {
+#pragma unroll 1
+        for (int s0 = 0; s0 < K; s0 += BT) {
+            ref_load<V, NS, BT, TL>(a, blk, i, K, wsrc, s0, q0);
+            use(s0, q0);
+        }
+        return;
+    }
+    FluxBatch<double, double, BT> q1;
+#pragma unroll 1
+    for (int s0 = 0; s0 < K; s0 += 2 * BT) {
+        if (s0 + BT < K) ref_load<V, NS, BT, TL>(a, blk, i, K, wsrc, s0 + BT, q1);
+        __builtin_amdgcn_sched_barrier(0);
+        use(s0, q0);
+        if (s0 + 2 * BT < K)
+            ref_load<V, NS, BT, TL>(a, blk, i, K, wsrc, s0 + 2 * BT, q0);
+        else if (wnext)
+            ref_load<V, NS, BT, TL>(a, blk, i, K, wnext, 0, q0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s0 + BT < K) use(s0 + BT, q1);
     }
 }
 
-template <int V, int NS, int HVK, bool RV, int BT, bool TL>
+template <int V, int NS, int HVK, bool RV, int BT, bool PF, bool TL>
 __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    const int64_t blk = remapped_block();
+    if (blk * kBlock >= a.N) return;  // whole block
+    const int K = NS ? NS : a.k;
+    const int64_t i_node = blk * kBlock + threadIdx.x;
+    // a thread without a node shadows the last node until the block-wide
+    // norm reduction, then leaves
+    const bool live = i_node < a.N;
+    const int64_t i = live ? i_node : a.N - 1;
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
+    FluxBatch<double, double, BT> q0;
+    if constexpr (PF) ref_load<V, NS, BT, TL>(a, blk, i, K, a.wx_s, 0, q0);
     __shared__ double wmax[kBlock / 64][4];
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
-    if (i_node == kNoBlock) return;  // whole block
-    // a thread without a node shadows the last node until the block-wide
-    // norm reduction, then leaves
-    const bool live = i_node >= 0;
+    stage_halo_a<V, TL>(a, blk, lds, rvres, pm, wmax);
     if (!rvres && !live) return;
-    const int64_t i = live ? i_node : a.N - 1;
-    const int K = NS ? NS : a.k;
     double du[V], gx[V], gy[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) du[v] = gx[v] = gy[v] = 0.0;
-    ref_pass<V, NS, RV, BT, 0, TL>(a, i, K, du, gx, lds);
-    ref_pass<V, NS, RV, BT, 1, TL>(a, i, K, du, gy, lds);
+    ref_pass<V, NS, RV, BT, PF, 0, TL>(a, blk, i, K, du, gx, lds, a.wx_s, q0, a.wy_s);
+    double ui[V], ad[V];  // the node's state and approx_du, in flight through the y pass
+    if constexpr (RV) {
+        load_state<V>(a.u, i, ui);
+        if (rvres) load_state<V>(a.approx, i, ad);
+    }
+    const bool fly = FLY && a.flyer_a;
+    ref_pass<V, NS, RV, BT, PF, 1, TL>(a, blk, i, K, du, gy, lds, a.wy_s, q0, fly ? a.hv_s : (TOM ? a.lap_s : nullptr));
     if constexpr (FLY) {
-        if (a.flyer_a) ref_pass<V, NS, false, BT, 2, TL>(a, i, K, du, nullptr, lds);
+        if (fly) ref_pass<V, NS, false, BT, PF, 2, TL>(a, blk, i, K, du, nullptr, lds, a.hv_s, q0, TOM ? a.lap_s : nullptr);
     }
     if constexpr (RV || TOM) {
         if constexpr (RV) {
-            double ui[V];
-            load_state<V>(a.u, i, ui);
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
-            const double e = node_viscosity(a, i, ui, du, ninf, &code);
+            const double e = node_viscosity(a, ui, du, ad, ninf, &code);
             a.eps[i] = e;
             a.epsc[i] = code;
             double g[2 * V];
@@ -742,7 +824,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
             double ll[V];
 #pragma unroll
             for (int v = 0; v < V; ++v) ll[v] = 0.0;
-            ref_pass<V, NS, false, BT, 3, TL>(a, i, K, ll, nullptr, lds);
+            ref_pass<V, NS, false, BT, PF, 3, TL>(a, blk, i, K, ll, nullptr, lds, a.lap_s, q0, nullptr);
             store_state<V>(a.L, i, ll);
         }
         store_state<V>(a.du, i, du);
@@ -757,64 +839,68 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
 // formed in FP64: sum_j w_ij F(u_j) ~= sum_j w_ij (F(u_j) - F(u_i)),
 // exact up to F(u_i) sum_j w_ij, which vanishes with the weights' row sums.
 // Weights FP32, neighbour indices as int16 offsets when the cloud allows.
-template <int V, int NS, int HVK, bool RV, bool D16, int BT, bool TL>
+template <int V, int NS, int HVK, bool RV, bool D16, int BT, bool PF, bool TL>
 __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    const int64_t blk = remapped_block();
+    if (blk * kBlock >= a.N) return;  // whole block
+    const int64_t N = a.N;
+    const int K = NS ? NS : a.k;
+    const int64_t i_node = blk * kBlock + threadIdx.x;
+    // a thread without a node shadows the last node until the block-wide
+    // norm reduction, then leaves
+    const bool live = i_node < N;
+    const int64_t i = live ? i_node : N - 1;
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
-    __shared__ double wmax[kBlock / 64][4];
-    const int64_t i_node = stage_halo_a<V, TL>(a, lds, rvres, pm, wmax);
-    if (i_node == kNoBlock) return;  // whole block
-    // a thread without a node shadows the last node until the block-wide
-    // norm reduction, then leaves
-    const bool live = i_node >= 0;
-    if (!rvres && !live) return;
-    const int64_t i = live ? i_node : a.N - 1;
-    const int64_t N = a.N;
-    const int K = NS ? NS : a.k;
-    double ui[V], fi1[V], fi2[V];
-    load_state<V>(a.u, i, ui);
-    flux_xy<V>(a.eq, ui, fi1, fi2);
-    float ax[V], ay[V], gx[V], gy[V], hh[V], ll[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) ax[v] = ay[v] = gx[v] = gy[v] = hh[v] = ll[v] = 0.0f;
-#pragma unroll 1
-    for (int s0 = 0; s0 < K; s0 += BT) {
-        int64_t jj[BT];
-        float2 ww[BT];
-        float hw32[BT], lw32[BT];
+    auto load = [&](int s0, FluxBatch<float2, float, BT>& q) {
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             const int s = s0 + b;
             if ((NS && NS % BT == 0) || s < K) {
-                const int64_t q = TL ? tm_pos(s, i, K) : (int64_t)s * N + i;
                 if constexpr (TL)
-                    jj[b] = a.la[q];
+                    q.j[b] = entry_of<TL>(a.la, blk, K, s, N, i);
                 else if constexpr (D16)
-                    jj[b] = i + (int64_t)a.didx[q];
+                    q.j[b] = (int32_t)i + (int32_t)entry_of<TL>(a.didx, blk, K, s, N, i);
                 else
-                    jj[b] = a.idx[q];
-                ww[b] = a.wxy32[q];
-                if constexpr (FLY) hw32[b] = a.hv32[q];
-                if constexpr (TOM) lw32[b] = a.lap32[q];
+                    q.j[b] = entry_of<TL>(a.idx, blk, K, s, N, i);
+                q.w[b] = entry_of<TL>(a.wxy32, blk, K, s, N, i);
+                if constexpr (FLY) q.hw[b] = entry_of<TL>(a.hv32, blk, K, s, N, i);
+                if constexpr (TOM) q.lw[b] = entry_of<TL>(a.lap32, blk, K, s, N, i);
             } else {
-                jj[b] = TL ? 0 : i;
-                ww[b] = make_float2(0.0f, 0.0f);
-                hw32[b] = lw32[b] = 0.0f;
+                q.j[b] = TL ? 0 : (int32_t)i;
+                q.w[b] = make_float2(0.0f, 0.0f);
+                q.hw[b] = q.lw[b] = 0.0f;
             }
         }
+    };
+    FluxBatch<float2, float, BT> q0;
+    if constexpr (PF) load(0, q0);
+    double ui[V], fi1[V], fi2[V], ad[V];
+    load_state<V>(a.u, i, ui);
+    if constexpr (RV) {
+        if (rvres) load_state<V>(a.approx, i, ad);
+    }
+    __shared__ double wmax[kBlock / 64][4];
+    stage_halo_a<V, TL>(a, blk, lds, rvres, pm, wmax);
+    if (!rvres && !live) return;
+    flux_xy<V>(a.eq, ui, fi1, fi2);
+    float ax[V], ay[V], gx[V], gy[V], hh[V], ll[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) ax[v] = ay[v] = gx[v] = gy[v] = hh[v] = ll[v] = 0.0f;
+    auto use = [&](const FluxBatch<float2, float, BT>& q) {
         // keep the batch's index and weight loads issued together, ahead of
         // the neighbour reads (the scheduler otherwise sinks each one to its use)
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!PF) __builtin_amdgcn_sched_barrier(0);
         double ub[BT][TL ? rec_len<V>() : V];
 #pragma unroll
-        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, jj[b], ub[b]);
+        for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, q.j[b], ub[b]);
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
-            const float2 w = ww[b];
+            const float2 w = q.w[b];
             const double* uj = ub[b];
             double f1[V], f2[V];
             flux_nb<V, TL>(a.eq, uj, f1, f2);
@@ -835,18 +921,19 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
                     }
                 }
                 if constexpr (FLY) {
-                    const float hw = hw32[b];
+                    const float hw = q.hw[b];
 #pragma unroll
                     for (int v = 0; v < V; ++v) hh[v] = fmaf(hw, dd[v], hh[v]);
                 }
                 if constexpr (TOM) {
-                    const float lw = lw32[b];
+                    const float lw = q.lw[b];
 #pragma unroll
                     for (int v = 0; v < V; ++v) ll[v] = fmaf(lw, dd[v], ll[v]);
                 }
             }
         }
-    }
+    };
+    for_batches<BT, PF>(K, q0, load, use);
     double du[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) du[v] = -(double)ax[v] - (double)ay[v];
@@ -862,7 +949,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
-            const double e = node_viscosity(a, i, ui, du, ninf, &code);
+            const double e = node_viscosity(a, ui, du, ad, ninf, &code);
             a.eps[i] = e;
             a.epsc[i] = code;
             double g[2 * V];
@@ -907,6 +994,16 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
 // wavefront (sb_off, sb_w), entries addressing halo records in LDS (lb:
 // halo positions; record q belongs to node hb_ids[hb_off[t] + q] and holds
 // its G (2V values) and / or L (V values)).
+// One batch of transposed entries: halo positions or rows, (Dx, Dy), lap.
+template <int TM, int BT>
+struct TransposeBatch {
+    using W2 = std::conditional_t<TM == 1, float2, double2>;
+    using W1 = std::conditional_t<TM == 1, float, double>;
+    int32_t r[BT];
+    W2 w[BT];
+    W1 wl[BT];
+};
+
 template <int V, int TM, int BT, bool TL, int GT>
 __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
 {
@@ -915,15 +1012,46 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
     constexpr int LU = HG ? 2 : 0;                   // unit of L in a record
     extern __shared__ double lds[];
     int64_t i, off = 0;
-    int lane = 0, W = 0;
+    int W = 0;
+    const int lane = threadIdx.x & 63;
     bool live;       // with a.stage_psum, threads past the last node stay for the block's sums
     int64_t blk;     // tile, or block of kBlock nodes
+    TransposeBatch<TM, BT> q0, q1;
+    auto load = [&](int e0, TransposeBatch<TM, BT>& q) {
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+            const int e = (e0 + b < W) ? e0 + b : e0;
+            const int64_t at = off + (int64_t)e * kSellC + lane;
+            if constexpr (TL)
+                q.r[b] = a.lb[at];
+            else
+                q.r[b] = a.trow[at];
+            if constexpr (HG) {
+                if constexpr (TM == 1)
+                    q.w[b] = TL ? a.twb32[at] : a.tw32[at];
+                else
+                    q.w[b] = TL ? a.twb[at] : a.tw[at];
+            }
+            if constexpr (HL) {
+                if constexpr (TM == 1)
+                    q.wl[b] = TL ? a.twl32[at] : a.tl32[at];
+                else
+                    q.wl[b] = TL ? a.twl[at] : a.tl[at];
+            }
+        }
+    };
     if constexpr (TL) {
         const int64_t t = remapped_block();
         if (t >= a.n_tiles) return;  // whole block
         blk = t;
         const int64_t h0 = a.hb_off[t];
         const int nh = (int)(a.hb_off[t + 1] - h0);
+        const int64_t sl = t * (kBlock / kSellC) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        off = a.sb_off[sl];
+        W = a.sb_w[sl];
+        i = t * kBlock + a.rowb[t * kBlock + threadIdx.x];
+        live = i < a.N;
+        if (W > 0) load(0, q0);
         for (int q = threadIdx.x; q < nh; q += kBlock) {
             const int64_t j = a.hb_ids[h0 + q];
             if constexpr (TM == 1) {  // FP32 records
@@ -954,16 +1082,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             }
         }
         __syncthreads();
-        const int pos = threadIdx.x;
-        i = t * kBlock + a.rowb[t * kBlock + pos];
-        live = i < a.N;
         if (!live && !a.stage_psum) return;
-        if (live) {
-            lane = pos & 63;
-            const int64_t sl = t * (kBlock / kSellC) + (pos >> 6);
-            off = a.sb_off[sl];
-            W = a.sb_w[sl];
-        }
     } else {
         i = remapped_node();
         if (i - threadIdx.x >= a.N) return;  // whole block
@@ -972,46 +1091,19 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
         if (!live && !a.stage_psum) return;
         if (live) {
             const int64_t slice = i >> 6;
-            lane = (int)(i & 63);
             off = a.sell_off[slice];
             W = a.sell_w[slice];
+            load(0, q0);
         }
     }
     double tx[V], ty[V], th[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) tx[v] = ty[v] = th[v] = 0.0;
-#pragma unroll 1
-    for (int e0 = 0; e0 < W; e0 += BT) {
-        int32_t r[BT];
-        double2 w[BT];
-        double wl[BT];
-#pragma unroll
-        for (int b = 0; b < BT; ++b) {
-            const int e = (e0 + b < W) ? e0 + b : e0;
-            const int64_t q = off + (int64_t)e * kSellC + lane;
-            if constexpr (TL)
-                r[b] = a.lb[q];
-            else
-                r[b] = a.trow[q];
-            if constexpr (HG) {
-                if constexpr (TM == 1) {
-                    const float2 w32 = TL ? a.twb32[q] : a.tw32[q];
-                    w[b] = make_double2((double)w32.x, (double)w32.y);
-                } else {
-                    w[b] = TL ? a.twb[q] : a.tw[q];
-                }
-            }
-            if constexpr (HL) {
-                if constexpr (TM == 1)
-                    wl[b] = (double)(TL ? a.twl32[q] : a.tl32[q]);
-                else
-                    wl[b] = TL ? a.twl[q] : a.tl[q];
-            }
-        }
+    auto use = [&](int e0, const TransposeBatch<TM, BT>& q) {
         double g0[BT][V], g1[BT][V], lv[BT][V];
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
-            const int64_t rb = r[b];
+            const int64_t rb = q.r[b];
             if constexpr (TM == 1) {
                 const float* ldsf = reinterpret_cast<const float*>(lds);
                 if constexpr (HG) {
@@ -1050,23 +1142,33 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             if (e0 + b >= W) continue;
+            const double wx = q.w[b].x, wy = q.w[b].y, wl = q.wl[b];
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 if constexpr (TM == 2) {
                     if constexpr (HG) {
-                        tx[v] = tx[v] + w[b].x * g0[b][v];
-                        ty[v] = ty[v] + w[b].y * g1[b][v];
+                        tx[v] = tx[v] + wx * g0[b][v];
+                        ty[v] = ty[v] + wy * g1[b][v];
                     }
-                    if constexpr (HL) th[v] = th[v] + wl[b] * lv[b][v];
+                    if constexpr (HL) th[v] = th[v] + wl * lv[b][v];
                 } else {
                     if constexpr (HG) {
-                        tx[v] = fma(w[b].x, g0[b][v], tx[v]);
-                        ty[v] = fma(w[b].y, g1[b][v], ty[v]);
+                        tx[v] = fma(wx, g0[b][v], tx[v]);
+                        ty[v] = fma(wy, g1[b][v], ty[v]);
                     }
-                    if constexpr (HL) th[v] = fma(wl[b], lv[b][v], th[v]);
+                    if constexpr (HL) th[v] = fma(wl, lv[b][v], th[v]);
                 }
             }
         }
+    };
+#pragma unroll 1
+    for (int e0 = 0; e0 < W; e0 += 2 * BT) {
+        if (e0 + BT < W) load(e0 + BT, q1);
+        __builtin_amdgcn_sched_barrier(0);
+        use(e0, q0);
+        if (e0 + 2 * BT < W) load(e0 + 2 * BT, q0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (e0 + BT < W) use(e0 + BT, q1);
     }
     double o[4] = {0.0, 0.0, 0.0, 0.0};  // the stored output (staged stages)
     if (live) {
@@ -2111,25 +2213,25 @@ constexpr int def_bt(int ns) { return ns ? 5 : 4; }
         else launch_k(c, 0, KERNEL<V, NS, 0, false, __VA_ARGS__>, G, B, lds, a);                         \
     } while (0)
 
-template <int V, int NS, int BT, bool TL>
+template <int V, int NS, int BT, bool PF, bool TL>
 static void launch_f64(mf_ctx* c, const RhsArgs& a, int hvk, bool rv, const dim3& G, size_t lds)
 {
     const dim3 B(kBlock);
-    MF_LAUNCH_HVK(k_rhs_f64, BT, TL);
+    MF_LAUNCH_HVK(k_rhs_f64, BT, PF, TL);
 }
 
-template <int V, int NS, int BT, bool D16, bool TL>
+template <int V, int NS, int BT, bool PF, bool D16, bool TL>
 static void launch_s32(mf_ctx* c, const RhsArgs& a, int hvk, bool rv, const dim3& G, size_t lds)
 {
     const dim3 B(kBlock);
-    MF_LAUNCH_HVK(k_rhs_s32, D16, BT, TL);
+    MF_LAUNCH_HVK(k_rhs_s32, D16, BT, PF, TL);
 }
 
-template <int V, int NS, int BT, bool TL>
+template <int V, int NS, int BT, bool PF, bool TL>
 static void launch_ref(mf_ctx* c, const RhsArgs& a, int hvk, bool rv, const dim3& G, size_t lds)
 {
     const dim3 B(kBlock);
-    MF_LAUNCH_HVK(k_rhs_ref, BT, TL);
+    MF_LAUNCH_HVK(k_rhs_ref, BT, PF, TL);
 }
 #undef MF_LAUNCH_HVK
 
@@ -2150,7 +2252,7 @@ static RhsArgs tile_major_args(const mf_ctx* c, const RhsArgs& a)
     return t;
 }
 
-template <int V, int NS, int BT>
+template <int V, int NS, int BT, bool PF>
 static void launch_flux_bt(mf_ctx* c, int prec, const RhsArgs& a_in, int hvk, bool rv, unsigned grid)
 {
     const dim3 G(grid);
@@ -2160,46 +2262,58 @@ static void launch_flux_bt(mf_ctx* c, int prec, const RhsArgs& a_in, int hvk, bo
     const size_t lds = tl ? (size_t)c->ha_max * rec_len<V>() * sizeof(double) : 0;  // halo records
     if (prec == MF_PREC_F64) {
         if (tl)
-            launch_f64<V, NS, BT, true>(c, a, hvk, rv, G, lds);
+            launch_f64<V, NS, BT, PF, true>(c, a, hvk, rv, G, lds);
         else
-            launch_f64<V, NS, BT, false>(c, a, hvk, rv, G, 0);
+            launch_f64<V, NS, BT, false, false>(c, a, hvk, rv, G, 0);
     } else if (prec == MF_PREC_F64_REF) {
         if (tl)
-            launch_ref<V, NS, BT, true>(c, a, hvk, rv, G, lds);
+            launch_ref<V, NS, BT, PF, true>(c, a, hvk, rv, G, lds);
         else
-            launch_ref<V, NS, BT, false>(c, a, hvk, rv, G, 0);
+            launch_ref<V, NS, BT, false, false>(c, a, hvk, rv, G, 0);
     } else if (tl) {
-        launch_s32<V, NS, BT, false, true>(c, a, hvk, rv, G, lds);
+        launch_s32<V, NS, BT, PF, false, true>(c, a, hvk, rv, G, lds);
     } else if (c->didx_ok) {
-        launch_s32<V, NS, BT, true, false>(c, a, hvk, rv, G, 0);
+        launch_s32<V, NS, BT, false, true, false>(c, a, hvk, rv, G, 0);
     } else {
-        launch_s32<V, NS, BT, false, false>(c, a, hvk, rv, G, 0);
+        launch_s32<V, NS, BT, false, false, false>(c, a, hvk, rv, G, 0);
     }
 }
 
-// Stencil batch sizes compiled per stencil size: the tuning value picks
-// one (it must divide the stencil size; 0 = the default, the first).  The
-// Tominec variants exist for the default only.
+// Variants compiled per stencil size, by the entries in flight per thread
+// (the tuning value): 3 and 5 are one batch at a time, 6 and 10 two batches
+// of 3 and 5 in turn (the next one in flight while the one at hand is used).
+// The Tominec variants exist for 5 and 10 only.
+// The default (0): up to two tiles per CU the few wavefronts cannot cover
+// each other's memory latency, and two batches in turn are faster; above,
+// their registers cost a resident workgroup.  Stencil kernel (us), one batch
+// of 5 / two of 3: 256^2 nodes (one tile per CU) reference order 14.6 / 14.4
+// (two of 5: 13.6), FP64 14.3 / 12.3, with Flyer 13.2 / 11.1, split-FP32
+// 11.6 / 11.1; 300^2 16.7 / 16.8, 16.2 / 15.1, 14.8 / 14.1, 13.4 / 13.6;
+// 512^2 37.3 / 37.4, 39.0 / 40.0, 34.2 / 33.4, 21.7 / 23.5.
 template <int V>
 static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool rv, unsigned grid)
 {
-    const int bt = (hvk & 2) ? 0 : c->tune_flux_batch[prec];
+    int bt = c->tune_flux_batch[prec];
+    const bool tl = c->tiles_a && !c->tm_dirty;
+    if (bt == 0 && tl && c->n_tiles <= c->cu_count) bt = prec == MF_PREC_F64_REF || c->k != 30 ? 10 : 6;
+    if (bt == 0 && tl && c->n_tiles <= 2 * c->cu_count && c->k == 30) bt = 6;
     switch (c->k) {
         case 15:
-            if (bt == 3) launch_flux_bt<V, 15, 3>(c, prec, a, hvk, rv, grid);
-            else launch_flux_bt<V, 15, 5>(c, prec, a, hvk, rv, grid);
+            if (bt == 10) launch_flux_bt<V, 15, 5, true>(c, prec, a, hvk, rv, grid);
+            else launch_flux_bt<V, 15, 5, false>(c, prec, a, hvk, rv, grid);
             break;
         case 20:
-            if (bt == 10) launch_flux_bt<V, 20, 10>(c, prec, a, hvk, rv, grid);
-            else launch_flux_bt<V, 20, 5>(c, prec, a, hvk, rv, grid);
+            if (bt == 10) launch_flux_bt<V, 20, 5, true>(c, prec, a, hvk, rv, grid);
+            else launch_flux_bt<V, 20, 5, false>(c, prec, a, hvk, rv, grid);
             break;
         case 30:
-            if (bt == 3) launch_flux_bt<V, 30, 3>(c, prec, a, hvk, rv, grid);
-            else if (bt == 6) launch_flux_bt<V, 30, 6>(c, prec, a, hvk, rv, grid);
-            else if (bt == 10) launch_flux_bt<V, 30, 10>(c, prec, a, hvk, rv, grid);
-            else launch_flux_bt<V, 30, 5>(c, prec, a, hvk, rv, grid);
+            if (hvk & 2) bt = bt == 6 || bt == 10 ? 10 : 0;
+            if (bt == 3) launch_flux_bt<V, 30, 3, false>(c, prec, a, hvk, rv, grid);
+            else if (bt == 6) launch_flux_bt<V, 30, 3, true>(c, prec, a, hvk, rv, grid);
+            else if (bt == 10) launch_flux_bt<V, 30, 5, true>(c, prec, a, hvk, rv, grid);
+            else launch_flux_bt<V, 30, 5, false>(c, prec, a, hvk, rv, grid);
             break;
-        default: launch_flux_bt<V, 0, 4>(c, prec, a, hvk, rv, grid); break;
+        default: launch_flux_bt<V, 0, 4, false>(c, prec, a, hvk, rv, grid); break;
     }
 }
 
@@ -2214,7 +2328,13 @@ static void launch_transpose_tl(mf_ctx* c, const RhsArgs& a, unsigned grid, size
     } else if (gt == 3) {
         launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 3>, G, B, lds, a);
     } else {
-        switch (c->tune_transpose_batch[TM]) {
+        // entries per batch, two batches in turn; the default: 8 while every
+        // tile has a CU of its own (256^2 nodes: 11.8 against 12.7 us for 4,
+        // split-FP32 9.7 against 11.1), 4 above, where 8 costs resident
+        // workgroups (512^2: 39.7 against 36.5)
+        int bt = c->tune_transpose_batch[TM];
+        if (bt == 0 && TL && c->n_tiles <= c->cu_count) bt = 8;
+        switch (bt) {
             case 2: launch_k(c, 1, k_rhs_transpose<4, TM, 2, TL, 1>, G, B, lds, a); break;
             case 8: launch_k(c, 1, k_rhs_transpose<4, TM, 8, TL, 1>, G, B, lds, a); break;
             default: launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 1>, G, B, lds, a); break;

@@ -19,7 +19,7 @@ import os
 
 from . import _lib as L
 
-FLUX_BATCHES = {15: (3, 5), 20: (5, 10), 30: (3, 5, 6, 10)}
+FLUX_BATCHES = {15: (5, 10), 20: (5, 10), 30: (3, 5, 6, 10)}
 TRANSPOSE_BATCHES = (2, 4, 8)
 PREC_NAMES = {L.MF_PREC_F64: "f64", L.MF_PREC_SPLIT32: "split32", L.MF_PREC_F64_REF: "f64_ref"}
 
