@@ -134,6 +134,8 @@ static void free_ops(mf_ctx* c)
     dfree(c->d_lap32);
     dfree(c->d_lap_s);
     dfree(c->d_tsrc);
+    dfree(c->d_tdeg);
+    c->d_tdeg = nullptr;
     dfree(c->d_tl);
     dfree(c->d_tl32);
     c->d_lap = c->d_lap_s = c->d_tl = nullptr;

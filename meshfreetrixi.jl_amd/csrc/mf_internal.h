@@ -121,6 +121,7 @@ struct mf_ctx {
     int32_t* d_trow = nullptr;
     double2* d_tw = nullptr;
     float2* d_tw32 = nullptr;
+    int32_t* d_tdeg = nullptr;  // entries of each column (rows of the transpose)
     int64_t* d_tsrc = nullptr;  // slot-major stencil position of each entry (-1: padding)
     double* d_tl = nullptr;     // lap of the transposed entries (Tominec)
     float* d_tl32 = nullptr;

@@ -23,7 +23,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <numeric>
+#include <cstdint>
 #include <type_traits>
 #include <vector>
 
@@ -163,171 +163,296 @@ static int upload(mf_ctx* c, T** dst, const std::vector<T>& v)
     return MF_OK;
 }
 
-// rec_b: doubles per phase-B halo record (G: 2 nvar, L: nvar), which
-// decides whether a tile's phase-B halo fits in LDS.
-int build_tiles(mf_ctx* c, bool want_b, int rec_b)
+// ------------------------------------------------- halos of the tiles
+// One workgroup per tile collects the distinct node ids of its entries in an
+// LDS hash table (open addressing), sorts the table (the empty slots last)
+// and looks every entry's position up in it by bisection.  Built on the
+// host, the tiles of 62,500 nodes took 70 ms, most of a new cloud's set-up
+// (bound by one core's cache misses); k_halo_a and k_halo_b take 0.11 ms each.
+constexpr int32_t kNoId = INT32_MAX;
+
+__device__ __forceinline__ void halo_clear(int32_t* tab, int T, int* cnt)
+{
+    for (int q = threadIdx.x; q < T; q += kTile) tab[q] = kNoId;
+    if (threadIdx.x == 0) *cnt = 0;
+    __syncthreads();
+}
+
+// Inserts id; at most cap + kTile ids enter the table (T above that, so a
+// probe always ends at an empty slot or the id).
+__device__ __forceinline__ void halo_insert(int32_t* tab, int T, int cap, int* cnt, int32_t id)
+{
+    uint32_t h = ((uint32_t)id * 2654435761u) >> (__clz(T) + 1);
+    for (;;) {
+        int32_t cur = reinterpret_cast<volatile int32_t*>(tab)[h];
+        if (cur == id) return;
+        if (cur == kNoId) {
+            if (*reinterpret_cast<volatile int*>(cnt) > cap) return;
+            cur = atomicCAS(&tab[h], kNoId, id);
+            if (cur == id) return;
+            if (cur == kNoId) {
+                atomicAdd(cnt, 1);
+                return;
+            }
+        }
+        h = (h + 1) & (uint32_t)(T - 1);
+    }
+}
+
+// Bitonic sort of the whole table, ascending.
+__device__ __forceinline__ void halo_sort(int32_t* tab, int T)
+{
+    for (int w = 2; w <= T; w <<= 1)
+        for (int d = w >> 1; d > 0; d >>= 1) {
+            for (int p = threadIdx.x; p < T / 2; p += kTile) {
+                const int lo = 2 * p - (p & (d - 1));  // bit d clear
+                const int32_t x = tab[lo], y = tab[lo + d];
+                if ((x > y) == ((lo & w) == 0)) {
+                    tab[lo] = y;
+                    tab[lo + d] = x;
+                }
+            }
+            __syncthreads();
+        }
+}
+
+__device__ __forceinline__ uint16_t halo_pos(const int32_t* tab, int n, int32_t id)
+{
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int m = (lo + hi) >> 1;
+        if (tab[m] < id)
+            lo = m + 1;
+        else
+            hi = m;
+    }
+    return (uint16_t)lo;
+}
+
+// The tile's ids (at t cap) and their number (above cap: the halo does not fit).
+__device__ __forceinline__ int halo_finish(int32_t* tab, int T, int cap, const int* cnt, int32_t* ids, int32_t* count,
+                                           int64_t t)
+{
+    __syncthreads();
+    const int n = *cnt;
+    if (threadIdx.x == 0) count[t] = n;
+    if (n > cap) return -1;
+    halo_sort(tab, T);
+    for (int q = threadIdx.x; q < n; q += kTile) ids[t * cap + q] = tab[q];
+    return n;
+}
+
+// Phase A: the union of the tile's stencils, and the tile-major positions of
+// the entries of both stencil copies (0 past the last node).
+__global__ __launch_bounds__(kTile) void k_halo_a(int64_t N, int K, const int32_t* idx, const int32_t* idx_s, int T,
+                                                  int cap, int32_t* ids, int32_t* count, uint16_t* la, uint16_t* la_s)
+{
+    extern __shared__ int32_t tab[];
+    __shared__ int cnt;
+    const int64_t t = blockIdx.x, i = t * kTile + threadIdx.x;
+    halo_clear(tab, T, &cnt);
+    if (i < N)
+        for (int s = 0; s < K; ++s) halo_insert(tab, T, cap, &cnt, idx[(int64_t)s * N + i]);
+    const int n = halo_finish(tab, T, cap, &cnt, ids, count, t);
+    if (n < 0) return;
+    for (int s = 0; s < K; ++s) {
+        const int64_t q = (t * K + s) * kTile + threadIdx.x;
+        la[q] = i < N ? halo_pos(tab, n, idx[(int64_t)s * N + i]) : 0;
+        la_s[q] = i < N ? halo_pos(tab, n, idx_s[(int64_t)s * N + i]) : 0;
+    }
+}
+
+// Phase B: the tile's rows by transposed degree, longest first (ties by
+// node; rows past the last node have degree 0), and the longest row of each
+// 64-row slice.
+__global__ __launch_bounds__(kTile) void k_rows_b(int64_t N, const int32_t* deg, uint8_t* rowb, int32_t* sw)
+{
+    __shared__ int32_t d[kTile], s[kTile];
+    const int64_t t = blockIdx.x, i = t * kTile + threadIdx.x;
+    const int r = threadIdx.x, mine = i < N ? deg[i] : 0;
+    d[r] = mine;
+    __syncthreads();
+    int at = 0;
+    for (int q = 0; q < kTile; ++q) at += d[q] > mine || (d[q] == mine && q < r);
+    rowb[t * kTile + at] = (uint8_t)r;
+    s[at] = mine;
+    __syncthreads();
+    if (r < kSlicesPerTile) sw[t * kSlicesPerTile + r] = s[r * kSellC];  // sorted: the slice's first row
+}
+
+// The union of the rows' entries, and each entry's halo position and source
+// in the slice layout (rows of the global transpose, already in ascending
+// caller index).
+__global__ __launch_bounds__(kTile) void k_halo_b(int64_t N, const int32_t* deg, const int64_t* toff,
+                                                  const int32_t* trow, const int64_t* tsrc, const uint8_t* rowb,
+                                                  const int64_t* soff, const int32_t* sw, int T, int cap, int32_t* ids,
+                                                  int32_t* count, uint16_t* lb, int64_t* src)
+{
+    extern __shared__ int32_t tab[];
+    __shared__ int cnt;
+    const int64_t t = blockIdx.x;
+    halo_clear(tab, T, &cnt);
+    {
+        const int64_t i = t * kTile + threadIdx.x;
+        if (i < N) {
+            const int64_t b = toff[i / kSellC] + i % kSellC;
+            const int n = deg[i];
+            for (int e = 0; e < n; ++e) halo_insert(tab, T, cap, &cnt, trow[b + (int64_t)e * kSellC]);
+        }
+    }
+    const int n = halo_finish(tab, T, cap, &cnt, ids, count, t);
+    if (n < 0) return;
+    const int p = threadIdx.x;
+    const int64_t i = t * kTile + rowb[t * kTile + p];
+    const int64_t sl = t * kSlicesPerTile + p / kSellC, o = soff[sl] + p % kSellC;
+    const int W = sw[sl], d = i < N ? deg[i] : 0;
+    const int64_t b = i < N ? toff[i / kSellC] + i % kSellC : 0;
+    for (int e = 0; e < W; ++e) {
+        const int64_t at = o + (int64_t)e * kSellC;
+        lb[at] = e < d ? halo_pos(tab, n, trow[b + (int64_t)e * kSellC]) : 0;
+        src[at] = e < d ? tsrc[b + (int64_t)e * kSellC] : -1;
+    }
+}
+
+// ids[off[t] + q] = tmp[t cap + q]
+__global__ void k_halo_pack(const int32_t* tmp, int cap, const int64_t* off, int32_t* ids)
+{
+    const int64_t t = blockIdx.x, o = off[t];
+    const int n = (int)(off[t + 1] - o);
+    for (int q = threadIdx.x; q < n; q += blockDim.x) ids[o + q] = tmp[t * cap + q];
+}
+
+static int halo_table(int cap)
+{
+    int T = 512;
+    while (T < cap + 2 * kTile) T *= 2;
+    return T;
+}
+
+// The halos' sizes (count) to offsets, the packed ids and the largest size;
+// fits = false if some tile's halo has more than cap ids.
+static int pack_halos(mf_ctx* c, int64_t nt, int cap, const int32_t* tmp, const int32_t* count, int64_t** off,
+                      int32_t** ids, int* hmax, int64_t* total, bool* fits)
+{
+    std::vector<int32_t> n(nt);
+    MF_HIP(c, hipMemcpyAsync(n.data(), count, sizeof(int32_t) * nt, hipMemcpyDeviceToHost, c->stream));
+    MF_HIP(c, hipStreamSynchronize(c->stream));
+    std::vector<int64_t> o(nt + 1, 0);
+    *hmax = 0;
+    for (int64_t t = 0; t < nt; ++t) {
+        *hmax = std::max<int>(*hmax, n[t]);
+        o[t + 1] = o[t] + n[t];
+    }
+    *total = o[nt];
+    *fits = *hmax <= cap;
+    if (!*fits) return MF_OK;
+    int rc;
+    if ((rc = upload(c, off, o)) || (rc = dalloc(c, ids, (size_t)o[nt]))) return rc;
+    hipLaunchKernelGGL(k_halo_pack, dim3((unsigned)nt), dim3(kTile), 0, c->stream, tmp, cap, *off, *ids);
+    MF_HIP(c, hipGetLastError());
+    MF_HIP(c, hipStreamSynchronize(c->stream));  // the offsets' host copy ends here
+    return MF_OK;
+}
+
+static int build_tiles_a(mf_ctx* c, int64_t nt, int32_t** tmp, int32_t** count)
 {
     const int64_t N = c->N;
     const int K = c->k;
-    const int V = c->nvar;
-    const int64_t nt = (N + kTile - 1) / kTile;
+    // phase A halo records: 6 doubles per node for Euler (state, v1, v2)
+    const int rec = c->nvar == 4 ? 6 : c->nvar;
+    const int cap = (int)(kTileLdsBytes / (rec * sizeof(double)));
+    const int T = halo_table(cap);
+    const size_t n_la = (size_t)nt * K * kTile;
     int rc;
-    std::vector<int32_t> idx((size_t)N * K), idx_s((size_t)N * K);
-    MF_HIP(c, hipMemcpyAsync(idx.data(), c->d_idx, sizeof(int32_t) * idx.size(), hipMemcpyDeviceToHost,
-                             c->stream));
-    MF_HIP(c, hipMemcpyAsync(idx_s.data(), c->d_idx_s, sizeof(int32_t) * idx_s.size(), hipMemcpyDeviceToHost,
-                             c->stream));
-    MF_HIP(c, hipStreamSynchronize(c->stream));
-    std::vector<int32_t> mark(N, -1);
-    std::vector<int32_t> ids;
-    ids.reserve(4 * kTile);
-
-    if (!c->tried_a) {
-        free_tiles(c);
-        c->tried_a = true;
-        std::vector<int64_t> off(nt + 1, 0);
-        std::vector<int32_t> all;
-        all.reserve((size_t)N * 2);
-        // tile-major (tm_pos): tile t's slot s at (t K + s) kTile
-        std::vector<uint16_t> la((size_t)nt * K * kTile, 0), la_s((size_t)nt * K * kTile, 0);
-        int hmax = 0;
-        bool fits = true;
-        for (int64_t t = 0; t < nt && fits; ++t) {
-            const int64_t i0 = t * kTile, i1 = std::min<int64_t>(N, i0 + kTile);
-            ids.clear();
-            for (int s = 0; s < K; ++s)
-                for (int64_t i = i0; i < i1; ++i) {
-                    const int32_t j = idx[(size_t)s * N + i];
-                    if (mark[j] < 0) {
-                        mark[j] = 0;
-                        ids.push_back(j);
-                    }
-                }
-            std::sort(ids.begin(), ids.end());
-            // phase A halo records: 6 doubles per node for Euler (state, v1, v2)
-            const size_t rec = (V == 4) ? 6 : (size_t)V;
-            if (ids.size() > 65535 || ids.size() * rec * sizeof(double) > kTileLdsBytes) fits = false;
-            for (size_t q = 0; q < ids.size(); ++q) mark[ids[q]] = (int32_t)q;
-            for (int s = 0; s < K; ++s)
-                for (int64_t i = i0; i < i1; ++i) {
-                    const size_t tq = (size_t)(t * K + s) * kTile + (size_t)(i - i0);
-                    la[tq] = (uint16_t)mark[idx[(size_t)s * N + i]];
-                    la_s[tq] = (uint16_t)mark[idx_s[(size_t)s * N + i]];
-                }
-            for (int32_t j : ids) mark[j] = -1;
-            hmax = std::max<int>(hmax, (int)ids.size());
-            all.insert(all.end(), ids.begin(), ids.end());
-            off[t + 1] = (int64_t)all.size();
-        }
-        if (!fits) return MF_OK;  // global-memory kernels
-        if ((rc = upload(c, &c->d_ha_off, off)) || (rc = upload(c, &c->d_ha_ids, all)) ||
-            (rc = upload(c, &c->d_la, la)) || (rc = upload(c, &c->d_la_s, la_s)))
-            return rc;
-        MF_HIP(c, hipStreamSynchronize(c->stream));
-        c->n_tiles = nt;
-        c->ha_max = hmax;
-        c->ha_total = (int64_t)all.size();
-        c->tiles_a = true;
-    }
-    if (!want_b || !c->tiles_a || c->tried_b) return MF_OK;
-    free_tiles_b(c);
-    c->tried_b = true;
-    c->tiles_b_rec = rec_b;
-
-    // transposed adjacency: the entries (j, s) with idx[s][j] = i, per row i,
-    // in ascending caller index of j
-    std::vector<int32_t> uid(N);
-    for (int64_t u = 0; u < N; ++u) uid[c->h_inv[u]] = (int32_t)u;
-    std::vector<int64_t> rp(N + 1, 0);
-    for (size_t q = 0; q < idx.size(); ++q) ++rp[idx[q] + 1];
-    for (int64_t i = 0; i < N; ++i) rp[i + 1] += rp[i];
-    std::vector<int64_t> ent(idx.size());  // slot-major position s*N + j
-    {
-        std::vector<int64_t> cur(rp.begin(), rp.end() - 1);
-        for (int s = 0; s < K; ++s)
-            for (int64_t j = 0; j < N; ++j) {
-                const int32_t i = idx[(size_t)s * N + j];
-                ent[cur[i]++] = (int64_t)s * N + j;
-            }
-    }
-    for (int64_t i = 0; i < N; ++i)
-        std::sort(ent.begin() + rp[i], ent.begin() + rp[i + 1], [&](int64_t a, int64_t b) {
-            const int32_t ua = uid[a % N], ub = uid[b % N];
-            return ua < ub || (ua == ub && a < b);
-        });
-    std::vector<int64_t> hoff(nt + 1, 0), soff(nt * kSlicesPerTile + 1, 0);
-    std::vector<int32_t> hall, sw(nt * kSlicesPerTile, 0);
-    std::vector<uint8_t> rowb((size_t)nt * kTile, 0);
-    std::vector<uint16_t> lb;
-    std::vector<int64_t> src;
-    int hmax = 0;
-    for (int64_t t = 0; t < nt; ++t) {
-        const int64_t i0 = t * kTile, i1 = std::min<int64_t>(N, i0 + kTile);
-        ids.clear();
-        for (int64_t i = i0; i < i1; ++i)
-            for (int64_t e = rp[i]; e < rp[i + 1]; ++e) {
-                const int32_t j = (int32_t)(ent[e] % N);
-                if (mark[j] < 0) {
-                    mark[j] = 0;
-                    ids.push_back(j);
-                }
-            }
-        std::sort(ids.begin(), ids.end());
-        if (ids.size() > 65535 || ids.size() * (size_t)rec_b * sizeof(double) > kTileLdsBytesB) {
-            for (int32_t j : ids) mark[j] = -1;
-            return MF_OK;  // global-memory transposed gather
-        }
-        for (size_t q = 0; q < ids.size(); ++q) mark[ids[q]] = (int32_t)q;
-        // rows by degree, longest first (rows past N have degree 0)
-        int order[kTile];
-        int deg[kTile];
-        for (int r = 0; r < kTile; ++r) {
-            order[r] = r;
-            deg[r] = (i0 + r < i1) ? (int)(rp[i0 + r + 1] - rp[i0 + r]) : 0;
-        }
-        std::stable_sort(order, order + kTile, [&](int a, int b) { return deg[a] > deg[b]; });
-        for (int p = 0; p < kTile; ++p) rowb[(size_t)t * kTile + p] = (uint8_t)order[p];
-        for (int w = 0; w < kSlicesPerTile; ++w) {
-            int W = 0;
-            for (int l = 0; l < kSellC; ++l) W = std::max(W, deg[order[w * kSellC + l]]);
-            const int64_t sl = t * kSlicesPerTile + w;
-            sw[sl] = W;
-            const size_t base = lb.size();
-            lb.resize(base + (size_t)W * kSellC, 0);
-            src.resize(base + (size_t)W * kSellC, -1);
-            for (int l = 0; l < kSellC; ++l) {
-                const int r = order[w * kSellC + l];
-                if (i0 + r >= i1) continue;
-                const int64_t i = i0 + r;
-                for (int64_t e = rp[i]; e < rp[i + 1]; ++e) {
-                    const size_t at = base + (size_t)(e - rp[i]) * kSellC + l;
-                    lb[at] = (uint16_t)mark[ent[e] % N];
-                    src[at] = ent[e];
-                }
-            }
-            soff[sl + 1] = (int64_t)lb.size();
-        }
-        for (int32_t j : ids) mark[j] = -1;
-        hmax = std::max<int>(hmax, (int)ids.size());
-        hall.insert(hall.end(), ids.begin(), ids.end());
-        hoff[t + 1] = (int64_t)hall.size();
-    }
-    if ((rc = upload(c, &c->d_hb_off, hoff)) || (rc = upload(c, &c->d_hb_ids, hall)) ||
-        (rc = upload(c, &c->d_sb_off, soff)) || (rc = upload(c, &c->d_sb_w, sw)) ||
-        (rc = upload(c, &c->d_rowb, rowb)) || (rc = upload(c, &c->d_lb, lb)) ||
-        (rc = upload(c, &c->d_tb_src, src)) || (rc = dalloc(c, &c->d_twb, lb.size())) ||
-        (rc = dalloc(c, &c->d_twb32, lb.size())))
+    if ((rc = dalloc(c, tmp, (size_t)nt * cap)) || (rc = dalloc(c, count, (size_t)nt)) ||
+        (rc = dalloc(c, &c->d_la, n_la)) || (rc = dalloc(c, &c->d_la_s, n_la)))
         return rc;
-    const int64_t ne = (int64_t)lb.size();
+    hipLaunchKernelGGL(k_halo_a, dim3((unsigned)nt), dim3(kTile), sizeof(int32_t) * T, c->stream, N, K, c->d_idx,
+                       c->d_idx_s, T, cap, *tmp, *count, c->d_la, c->d_la_s);
+    MF_HIP(c, hipGetLastError());
+    bool fits;
+    int hmax;
+    if ((rc = pack_halos(c, nt, cap, *tmp, *count, &c->d_ha_off, &c->d_ha_ids, &hmax, &c->ha_total, &fits))) return rc;
+    if (!fits) {  // global-memory kernels
+        dfree(c->d_la);
+        dfree(c->d_la_s);
+        c->d_la = c->d_la_s = nullptr;
+        return MF_OK;
+    }
+    c->n_tiles = nt;
+    c->ha_max = hmax;
+    c->tiles_a = true;
+    return MF_OK;
+}
+
+static int build_tiles_b(mf_ctx* c, int64_t nt, int rec_b, int32_t** tmp, int32_t** count)
+{
+    const int64_t N = c->N;
+    const int cap = (int)(kTileLdsBytesB / (rec_b * sizeof(double)));
+    const int T = halo_table(cap);
+    const int64_t nsl = nt * kSlicesPerTile;
+    int rc;
+    if ((rc = dalloc(c, tmp, (size_t)nt * cap)) || (rc = dalloc(c, count, (size_t)nt)) ||
+        (rc = dalloc(c, &c->d_rowb, (size_t)nt * kTile)) || (rc = dalloc(c, &c->d_sb_w, (size_t)nsl)))
+        return rc;
+    hipLaunchKernelGGL(k_rows_b, dim3((unsigned)nt), dim3(kTile), 0, c->stream, N, c->d_tdeg, c->d_rowb, c->d_sb_w);
+    MF_HIP(c, hipGetLastError());
+    std::vector<int32_t> sw(nsl);
+    MF_HIP(c, hipMemcpyAsync(sw.data(), c->d_sb_w, sizeof(int32_t) * nsl, hipMemcpyDeviceToHost, c->stream));
+    MF_HIP(c, hipStreamSynchronize(c->stream));
+    std::vector<int64_t> soff(nsl + 1, 0);
+    for (int64_t s = 0; s < nsl; ++s) soff[s + 1] = soff[s] + (int64_t)sw[s] * kSellC;
+    const int64_t ne = soff[nsl];
+    if ((rc = upload(c, &c->d_sb_off, soff)) || (rc = dalloc(c, &c->d_lb, (size_t)ne)) ||
+        (rc = dalloc(c, &c->d_tb_src, (size_t)ne)))
+        return rc;
+    hipLaunchKernelGGL(k_halo_b, dim3((unsigned)nt), dim3(kTile), sizeof(int32_t) * T, c->stream, N, c->d_tdeg,
+                       c->d_sell_off, c->d_trow, c->d_tsrc, c->d_rowb, c->d_sb_off, c->d_sb_w, T, cap, *tmp, *count,
+                       c->d_lb, c->d_tb_src);
+    MF_HIP(c, hipGetLastError());
+    bool fits;
+    int hmax;
+    if ((rc = pack_halos(c, nt, cap, *tmp, *count, &c->d_hb_off, &c->d_hb_ids, &hmax, &c->hb_total, &fits))) return rc;
+    if (!fits) return MF_OK;  // global-memory transposed gather
+    if ((rc = dalloc(c, &c->d_twb, (size_t)ne)) || (rc = dalloc(c, &c->d_twb32, (size_t)ne))) return rc;
     hipLaunchKernelGGL(k_fill_tile_weights, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, c->stream, ne,
                        c->d_tb_src, c->d_wxy, c->d_twb, c->d_twb32);
     MF_HIP(c, hipGetLastError());
     MF_HIP(c, hipStreamSynchronize(c->stream));
     c->hb_max = hmax;
-    c->hb_total = (int64_t)hall.size();
     c->nb_entries = ne;
     c->tiles_b = true;
     return MF_OK;
+}
+
+// rec_b: doubles per phase-B halo record (G: 2 nvar, L: nvar), which
+// decides whether a tile's phase-B halo fits in LDS.  Phase B needs the
+// global transpose.
+int build_tiles(mf_ctx* c, bool want_b, int rec_b)
+{
+    const int64_t nt = (c->N + kTile - 1) / kTile;
+    int rc = MF_OK;
+    int32_t *tmp = nullptr, *count = nullptr;
+    if (!c->tried_a) {
+        free_tiles(c);
+        c->tried_a = true;
+        rc = build_tiles_a(c, nt, &tmp, &count);
+        if (rc) (void)hipStreamSynchronize(c->stream);  // nothing in flight reads them
+        dfree(tmp);
+        dfree(count);
+        if (rc) return rc;
+    }
+    if (!want_b || !c->tiles_a || c->tried_b) return MF_OK;
+    if (!c->have_T) return fail(c, MF_ERR_STATE, "tiles: no transposed operator");
+    free_tiles_b(c);
+    c->tried_b = true;
+    c->tiles_b_rec = rec_b;
+    tmp = count = nullptr;
+    rc = build_tiles_b(c, nt, rec_b, &tmp, &count);
+    if (rc) (void)hipStreamSynchronize(c->stream);
+    dfree(tmp);
+    dfree(count);
+    return rc;
 }
 
 }  // namespace mf
