@@ -14,8 +14,6 @@
 
 namespace mf {
 
-int bc_pass_homog(mf_ctx* c, double* u);
-int bc_pass_state(mf_ctx* c, double* u, double dt_off);
 int ensure_state(mf_ctx* c);
 int run_rhs(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off, const StageOut& st);
 
@@ -333,7 +331,7 @@ int mf_rhs_vjp(mf_ctx* c, double t)
     if (c->visc_mode != MF_VISC_NONE || c->hv_gamma != 0.0 || c->tom_gamma != 0.0 || c->igr_alpha != 0.0)
         return fail(c, MF_ERR_UNSUPPORTED, "mf_rhs_vjp: sources have no adjoint in this build");
     if ((rc = prepare_vjp(c))) return rc;
-    if ((rc = run_set_time(c, t, -1))) return rc;
+    const HostTime time(c, t);
     // J is evaluated at P u: boundary pass on a copy of u
     if ((rc = copy_state(c, c->d_S, c->d_buf[MF_BUF_U]))) return rc;
     if ((rc = bc_pass_state(c, c->d_S, 0.0))) return rc;
@@ -387,12 +385,18 @@ int mf_ssprk33_vjp(mf_ctx* c, double t0, double dt, int n_steps, int checkpoint_
     std::vector<double> tn(n_steps + 1);
     tn[0] = t0;
     for (int n = 0; n < n_steps; ++n) tn[n + 1] = tn[n] + dt;
-    // one forward step from raw state X (mutated to X'), stages into S and T
-    // (left post-boundary), result (raw) into Y
+    HostTime time(c, t0);
+    // one forward step from state X, stages into S and T (left
+    // post-boundary), result into Y.  With hand every state is written with
+    // the first boundary pass of the rhs! that reads it (X with that of this
+    // step), as the stages of mf_ssprk33; otherwise X and Y are raw.
+    const bool hand = !(c->have_bc && c->bc.multi);
     auto fwd = [&](int n, double* X, double* S, double* T, double* Y) -> int {
         int r2;
-        if ((r2 = run_set_time(c, tn[n], -1))) return r2;
+        time.set(tn[n]);
         StageOut s1;
+        s1.handed_in = s1.handed_out = hand;
+        s1.out_dt_off = dt;
         s1.kind = ST_FSAL;
         s1.dt = dt;
         s1.out = S;
@@ -402,20 +406,25 @@ int mf_ssprk33_vjp(mf_ctx* c, double t0, double dt, int n_steps, int checkpoint_
         s2.dt = dt;
         s2.uprev = X;
         s2.out = T;
+        s2.handed_in = s2.handed_out = hand;
+        s2.out_dt_off = dt / 2.0;
         if ((r2 = run_rhs(c, MF_PREC_F64, S, c->d_buf[MF_BUF_DU], dt, s2))) return r2;
         StageOut s3;
         s3.kind = ST_THREE;
         s3.dt = dt;
         s3.uprev = X;
         s3.out = Y;
+        s3.handed_in = s3.handed_out = hand;
+        s3.out_dt_off = dt;  // Y's next step starts at tn[n] + dt
         return run_rhs(c, MF_PREC_F64, T, c->d_buf[MF_BUF_DU], dt / 2.0, s3);
     };
     // tape of segment step n (first step n0): X at 3 (n - n0), S and T after it
     auto tape_x = [&](int n, int n0) { return tape + (int64_t)(3 * (n - n0)) * NV; };
-    // forward pass with checkpoints (raw states at steps 0, C, 2C, ...); the
+    // forward pass with checkpoints (states at steps 0, C, 2C, ...); the
     // last segment keeps its tape, so the reverse sweep does not recompute it
     const int last0 = (nck - 1) * C;
     if ((rc = copy_state(c, W0, c->d_buf[MF_BUF_U]))) return rc;
+    if (hand && (rc = bc_pass_state(c, W0, 0.0))) return rc;
     for (int n = 0; n < last0; ++n) {
         if (n % C == 0 && (rc = copy_state(c, buf(n / C), W0))) return rc;
         if ((rc = fwd(n, W0, tape, tape + NV, W1))) return rc;
@@ -427,8 +436,8 @@ int mf_ssprk33_vjp(mf_ctx* c, double t0, double dt, int n_steps, int checkpoint_
         if ((rc = fwd(n, Xn, Xn + NV, Xn + 2 * NV, n + 1 < n_steps ? tape_x(n + 1, last0) : W1))) return rc;
     }
     // loss on the final state (W1) after its boundary pass (the last FSAL call)
-    if ((rc = run_set_time(c, tn[n_steps], -1))) return rc;
-    if ((rc = bc_pass_state(c, W1, 0.0))) return rc;
+    time.set(tn[n_steps]);
+    if (!hand && (rc = bc_pass_state(c, W1, 0.0))) return rc;
     double* d_loss = W0;
     hipLaunchKernelGGL(k_loss, dim3(1), dim3(1024), 0, c->stream, c->N, c->nvar, W1, Ub, d_loss);
     MF_HIP(c, hipGetLastError());

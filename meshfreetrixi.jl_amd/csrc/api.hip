@@ -103,8 +103,6 @@ PhsTable phs_table(int p, int k)
     return t;
 }
 
-int bc_pass_homog(mf_ctx* c, double* u);
-int bc_pass_state(mf_ctx* c, double* u, double dt_off);
 
 static void free_ops(mf_ctx* c)
 {
@@ -194,19 +192,16 @@ static void free_state(mf_ctx* c)
 static void free_bc(mf_ctx* c)
 {
     dfree(c->bc.bidx);
-    dfree(c->bc.btag);
     dfree(c->bc.bnormal);
     dfree(c->bc.btable);
     dfree(c->bc.flag);
     dfree(c->bc.entry);
     dfree(c->bc.ecode);
-    dfree(c->bc.d_kind);
-    dfree(c->bc.d_kind_slip);
-    dfree(c->bc.d_fn);
     dfree(c->bc.d_params);
-    c->bc.d_kind = c->bc.d_kind_slip = c->bc.d_fn = nullptr;
+    dfree(c->d_sraw);
+    c->d_sraw = nullptr;
     c->bc.d_params = nullptr;
-    c->bc.bidx = c->bc.btag = c->bc.entry = c->bc.ecode = nullptr;
+    c->bc.bidx = c->bc.entry = c->bc.ecode = nullptr;
     c->bc.bnormal = c->bc.btable = nullptr;
     c->bc.flag = nullptr;
     c->have_bc = false;
@@ -822,6 +817,17 @@ int mf_weights_ragged_get(mf_ctx* c, double* wx, double* wy)
     return MF_OK;
 }
 
+// The stored FSAL stage as it was before its next boundary pass (which the
+// step that wrote it applied): before the boundary conditions change, or for
+// steps that run that pass themselves.  With the residual viscosity the
+// stage stays as it is (its sums go with it).
+static int raw_fsal(mf_ctx* c)
+{
+    if (!c->fsal_valid || !c->fsal_handed || c->fsal_sums) return MF_OK;
+    c->fsal_handed = false;
+    return c->d_sraw ? run_restore_raw(c, c->d_S) : MF_OK;
+}
+
 int mf_set_equations(mf_ctx* c, int equations, double p0, double p1)
 {
     int rc = check_ctx(c);
@@ -835,6 +841,7 @@ int mf_set_equations(mf_ctx* c, int equations, double p0, double p1)
     } else {
         return fail(c, MF_ERR_ARGUMENT, "mf_set_equations: unknown equations");
     }
+    if ((rc = raw_fsal(c))) return rc;  // boundary values depend on gamma
     MF_HIP(c, hipStreamSynchronize(c->stream));
     if (nv != c->nvar) {
         free_state(c);
@@ -856,6 +863,7 @@ int mf_set_boundary(mf_ctx* c, int n_tags, const int32_t* tag_ptr, const int32_t
     if (rc) return rc;
     if (c->N == 0) return fail(c, MF_ERR_STATE, "mf_set_boundary: no points");
     if (n_tags < 0 || n_tags > kMaxTags) return fail(c, MF_ERR_ARGUMENT, "mf_set_boundary: too many tags");
+    if ((rc = raw_fsal(c))) return rc;
     MF_HIP(c, hipStreamSynchronize(c->stream));
     free_bc(c);
     free_graph(c);
@@ -912,25 +920,16 @@ int mf_set_boundary(mf_ctx* c, int n_tags, const int32_t* tag_ptr, const int32_t
     }
     b.tag_ptr[n_tags] = nb;
     b.nb = nb;
-    if ((rc = dalloc(c, &b.bidx, nb)) || (rc = dalloc(c, &b.btag, nb)) || (rc = dalloc(c, &b.bnormal, 2 * (size_t)nb)) ||
+    if ((rc = dalloc(c, &b.bidx, nb)) || (rc = dalloc(c, &b.bnormal, 2 * (size_t)nb)) ||
         (rc = dalloc(c, &b.btable, (size_t)nb * 4)) || (rc = dalloc(c, &b.flag, c->N)) || (rc = dalloc(c, &b.entry, c->N)) ||
         (rc = dalloc(c, &b.ecode, std::max(nb, 1))) ||
-        (rc = dalloc(c, &b.d_kind, n_tags)) || (rc = dalloc(c, &b.d_kind_slip, n_tags)) ||
-        (rc = dalloc(c, &b.d_fn, n_tags)) || (rc = dalloc(c, &b.d_params, 8 * (size_t)n_tags)))
+        (rc = dalloc(c, &b.d_params, 8 * (size_t)n_tags)))
         return rc;
-    std::vector<int32_t> kind_slip(n_tags);
-    for (int g = 0; g < n_tags; ++g)
-        kind_slip[g] = b.tag_kind[g] == MF_BC_SLIP_WALL ? MF_BC_SLIP_WALL : MF_BC_DO_NOTHING;
-    MF_HIP(c, hipMemcpyAsync(b.d_kind, b.tag_kind.data(), sizeof(int32_t) * n_tags, hipMemcpyHostToDevice, c->stream));
-    MF_HIP(c, hipMemcpyAsync(b.d_kind_slip, kind_slip.data(), sizeof(int32_t) * n_tags, hipMemcpyHostToDevice,
-                             c->stream));
-    MF_HIP(c, hipMemcpyAsync(b.d_fn, b.tag_fn.data(), sizeof(int32_t) * n_tags, hipMemcpyHostToDevice, c->stream));
     MF_HIP(c, hipMemcpyAsync(b.d_params, b.tag_params.data(), sizeof(double) * 8 * n_tags, hipMemcpyHostToDevice,
                              c->stream));
     std::vector<double> nrm(2 * (size_t)std::max(nb, 1), 0.0);
     if (normals) std::copy(normals, normals + 2 * (size_t)nb, nrm.begin());
     MF_HIP(c, hipMemcpyAsync(b.bidx, bnode.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, c->stream));
-    MF_HIP(c, hipMemcpyAsync(b.btag, btag.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, c->stream));
     // each entry's kind, value function and tag in one word: the fused
     // first pass (sum pass, stage hand-over) reads them with one load
     std::vector<int32_t> ecode(std::max(nb, 1), 0);
@@ -953,6 +952,7 @@ int mf_set_boundary_values(mf_ctx* c, const double* values)
     if (rc) return rc;
     if (!c->have_bc) return fail(c, MF_ERR_STATE, "mf_set_boundary_values: no boundary");
     if (!values) return fail(c, MF_ERR_ARGUMENT, "mf_set_boundary_values: null values");
+    if ((rc = raw_fsal(c))) return rc;
     MF_HIP(c, hipMemcpyAsync(c->bc.btable, values, sizeof(double) * c->bc.nb * c->nvar, hipMemcpyHostToDevice,
                              c->stream));
     MF_HIP(c, hipStreamSynchronize(c->stream));
@@ -1201,7 +1201,7 @@ int mf_rhs(mf_ctx* c, double t, int precision)
     int rc = check_ctx(c);
     if (rc) return rc;
     if ((rc = prepare_rhs(c))) return rc;
-    if ((rc = run_set_time(c, t, -1))) return rc;
+    const HostTime time(c, t);
     StageOut none;
     if ((rc = run_rhs(c, precision, c->d_buf[MF_BUF_U], c->d_buf[MF_BUF_DU], 0.0, none))) return rc;
     c->fsal_valid = false;
@@ -1310,21 +1310,26 @@ int mf_set_stage_limiter(mf_ctx* c, int n, const double* thresholds, const int32
     return MF_OK;
 }
 
-// Whether the stages of mf_ssprk33 hand each other the next rhs!'s first
-// boundary pass and sums (the residual viscosity's transposed kernel
-// writes each stage; no stage limiter runs between them).
-static bool stage_sums(const mf_ctx* c, bool limiter)
+// Whether the stages of mf_ssprk33 are handed over: the kernel that writes a
+// stage applies the next rhs!'s first boundary pass to it (and, with the
+// residual viscosity, leaves its sums), so that rhs! starts without a launch
+// of its own for them.  Not with a stage limiter, which runs between the two
+// on the stage as it is, nor where a node carries several conditions.
+static bool stage_handover(const mf_ctx* c, bool limiter)
 {
-    return c->visc_mode == MF_VISC_RESIDUAL && !limiter && c->igr_alpha == 0.0 && c->d_stage_psum &&
-           !(c->have_bc && c->bc.multi) && !(c->tiles_b && c->n_tiles != (c->N + kBlock - 1) / kBlock);
+    if (limiter || c->igr_alpha != 0.0 || (c->have_bc && c->bc.multi)) return false;
+    return c->visc_mode != MF_VISC_RESIDUAL ||
+           (c->d_stage_psum && !(c->tiles_b && c->n_tiles != (c->N + kBlock - 1) / kBlock));
 }
 
 // One SSPRK33 step on U with the FSAL stage S = U + dt f(U) already formed.
-// With sums, every rhs! of the step takes its input's boundary pass and
-// sums from the rhs! before it and leaves them for the next: T's and U's
-// at this step's stage times t + dt/2 and t + dt, S's at the next step's
-// t + dt (the time is advanced after the last rhs!).
-static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history, bool sums)
+// With hand, every rhs! of the step takes its input with its first boundary
+// pass (and sums) from the rhs! before it and leaves the same for the next:
+// T's and U's at this step's stage times t + dt/2 and t + dt, S's at the
+// next step's t_next + dt.  The time moves on in the stage kernels: the
+// second stage writes t_next = t + dt, the last makes it t (with the history
+// callback, which needs both, the callback does).
+static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history, bool hand)
 {
     int rc;
     auto limit = [&](double* u) -> int {
@@ -1342,8 +1347,10 @@ static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history
     s2.dt = dt;
     s2.uprev = U;
     s2.out = c->d_T;
-    s2.sums_in = s2.sums_out = sums;
+    s2.handed_in = s2.handed_out = hand;
     s2.out_dt_off = dt / 2.0;
+    s2.time = StageOut::kTimeNext;
+    s2.u_dead = true;
     if ((rc = run_rhs(c, prec, c->d_S, c->d_buf[MF_BUF_DU], dt, s2))) return rc;
     if ((rc = limit(c->d_T))) return rc;
     StageOut s3;
@@ -1351,23 +1358,22 @@ static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history
     s3.dt = dt;
     s3.uprev = U;
     s3.out = U;
-    s3.sums_in = s3.sums_out = sums;
+    s3.handed_in = s3.handed_out = hand;
     s3.out_dt_off = dt;
+    s3.u_dead = true;
     if ((rc = run_rhs(c, prec, c->d_T, c->d_buf[MF_BUF_DU], dt / 2.0, s3))) return rc;
     if ((rc = limit(U))) return rc;
     StageOut s1;
     s1.kind = ST_FSAL;
     s1.dt = dt;
     s1.out = c->d_S;
-    s1.sums_in = s1.sums_out = sums;
-    s1.out_t_adv = dt;
+    s1.handed_in = s1.handed_out = hand;
+    s1.keep_raw = true;
+    s1.out_t_next = true;
     s1.out_dt_off = dt;
+    if (!history) s1.time = StageOut::kTimeAdvance;
     if ((rc = run_rhs(c, prec, U, c->d_buf[MF_BUF_DU], dt, s1))) return rc;
-    if (history) {
-        if ((rc = run_history(c, U, 0, dt))) return rc;  // also advances the time
-    } else if ((rc = run_advance_time(c, dt))) {
-        return rc;
-    }
+    if (history) return run_history(c, U, 0, dt);  // also advances the time
     return MF_OK;
 }
 
@@ -1379,16 +1385,26 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
     if ((rc = prepare_rhs(c))) return rc;
     const bool limiter = (flags & MF_STEP_LIMITER) && c->lim_n > 0;
     const int gflags = flags & ~MF_STEP_NOSYNC;  // what the captured step depends on
-    const bool history = (flags & MF_STEP_HISTORY) && c->visc_mode == MF_VISC_RESIDUAL;
-    const bool sums = stage_sums(c, limiter);
+    const bool residual = c->visc_mode == MF_VISC_RESIDUAL;
+    const bool history = (flags & MF_STEP_HISTORY) && residual;
+    const bool hand = stage_handover(c, limiter);
+    if (hand && !residual && c->have_bc && !c->d_sraw &&
+        (rc = dalloc(c, &c->d_sraw, (size_t)c->bc.nb * kMaxVar)))
+        return rc;
     if (resume) {
         if (!c->fsal_valid || c->fsal_dt != dt)
             return fail(c, MF_ERR_STATE, "mf_ssprk33: resume needs the previous call's state and the same dt");
         // with the residual viscosity the stored FSAL stage carries the
         // next boundary pass and sums exactly when no stage limiter runs
-        if (c->fsal_sums != sums)
+        if (c->fsal_sums != (hand && residual))
             return fail(c, MF_ERR_STATE,
                         "mf_ssprk33: resume needs the previous call's stage limiter and viscosity settings");
+        if (n_steps == 0) {  // nothing to do: the stage stays as it is
+            if (!(flags & MF_STEP_NOSYNC)) MF_HIP(c, hipStreamSynchronize(c->stream));
+            return MF_OK;
+        }
+        if (!hand && (rc = raw_fsal(c))) return rc;
+        if (hand && !c->fsal_handed && (rc = bc_pass_state(c, c->d_S, dt))) return rc;
     } else {
         if ((rc = run_set_time(c, t0, 0))) return rc;
         if (history && (rc = run_history(c, c->d_buf[MF_BUF_U], 1))) return rc;
@@ -1396,7 +1412,8 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
         s1.kind = ST_FSAL;
         s1.dt = dt;
         s1.out = c->d_S;
-        s1.sums_out = sums;  // for the first step's rhs! at t0 + dt
+        s1.handed_out = hand;  // for the first step's rhs! at t0 + dt
+        s1.keep_raw = true;
         s1.out_dt_off = dt;
         if ((rc = run_rhs(c, precision, c->d_buf[MF_BUF_U], c->d_buf[MF_BUF_DU], 0.0, s1))) return rc;
         c->host_success_iter = 0;
@@ -1407,7 +1424,7 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
         auto capture = [&](int steps, hipGraph_t* graph, hipGraphExec_t* exec) -> int {
             MF_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             int r = MF_OK;
-            for (int s = 0; s < steps && r == MF_OK; ++s) r = ssprk_step(c, dt, precision, limiter, history, sums);
+            for (int s = 0; s < steps && r == MF_OK; ++s) r = ssprk_step(c, dt, precision, limiter, history, hand);
             hipGraph_t g = nullptr;
             hipError_t e = hipStreamEndCapture(c->stream, &g);
             if (r) {
@@ -1420,14 +1437,14 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
             return MF_OK;
         };
         if (!c->step_exec || c->graph_prec != precision || c->graph_flags != gflags || c->graph_dt != dt ||
-            c->graph_sums != sums) {
+            c->graph_hand != hand) {
             free_graph(c);
             MF_HIP(c, hipStreamSynchronize(c->stream));
             if ((rc = capture(1, &c->step_graph, &c->step_exec))) return rc;
             c->graph_prec = precision;
             c->graph_flags = gflags;
             c->graph_dt = dt;
-            c->graph_sums = sums;
+            c->graph_hand = hand;
         }
         if (n_steps >= kGraphSteps && !c->multi_exec &&
             (rc = capture(kGraphSteps, &c->multi_graph, &c->multi_exec)))
@@ -1437,10 +1454,11 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
         for (; n < n_steps; ++n) MF_HIP(c, hipGraphLaunch(c->step_exec, c->stream));
     } else {
         for (int n = 0; n < n_steps; ++n)
-            if ((rc = ssprk_step(c, dt, precision, limiter, history, sums))) return rc;
+            if ((rc = ssprk_step(c, dt, precision, limiter, history, hand))) return rc;
     }
     c->fsal_dt = dt;
-    c->fsal_sums = sums;
+    c->fsal_sums = hand && residual;
+    c->fsal_handed = hand;
     c->host_success_iter += n_steps;
     c->fsal_valid = true;
     if (!(flags & MF_STEP_NOSYNC)) MF_HIP(c, hipStreamSynchronize(c->stream));

@@ -20,6 +20,7 @@ constexpr int kMaxStencilM = 64;  // saddle systems up to 64 x 64 (one wavefront
 // current time, history weights and success_iter at replay.
 struct StepScalars {
     double t;                    // integrator time t_n
+    double t_next;               // t_n + dt, written by the step's second stage
     double time_hist[kMaxHist];  // most recent first
     double tw[kMaxHist];         // time-derivative weights
     double norms[2 * kMaxVar];   // mean(u), ninf of |u - mean| (residual viscosity)
@@ -54,7 +55,6 @@ struct BcDev {
     int any_slip;
     int multi;  // some node belongs to more than one tag
     int32_t* bidx = nullptr;     // nb
-    int32_t* btag = nullptr;     // nb
     double* bnormal = nullptr;   // 2 nb
     double* btable = nullptr;    // nvar nb
     uint8_t* flag = nullptr;     // N: bit0 Dirichlet, bit1 slip
@@ -64,9 +64,6 @@ struct BcDev {
     std::vector<int32_t> tag_fn;
     std::vector<int32_t> tag_ptr;
     std::vector<double> tag_params;    // 8 per tag
-    int32_t* d_kind = nullptr;         // ntags: tag kinds
-    int32_t* d_kind_slip = nullptr;    // ntags: slip walls kept, other kinds as do-nothing
-    int32_t* d_fn = nullptr;           // ntags: value functions
     double* d_params = nullptr;        // 8 ntags: value-function parameters
 };
 
@@ -167,8 +164,13 @@ struct mf_ctx {
     mf::StepScalars* d_sc = nullptr;
     int host_success_iter = 0;
     bool fsal_valid = false;
-    bool fsal_sums = false;   // the stored FSAL stage carries its next boundary pass and sums
-    bool graph_sums = false;  // the captured step passes them between stages
+    bool fsal_sums = false;    // the stored FSAL stage carries its sums (residual viscosity)
+    bool fsal_handed = false;  // and has had its next boundary pass
+    bool graph_hand = false;   // the captured step hands its stages over
+    double* d_sraw = nullptr;  // the FSAL stage's boundary entries before that pass (nvar each)
+    // the time of eager calls, by value (HostTime)
+    bool host_time = false;
+    double t_host = 0.0;
 
     // stage limiter
     int lim_n = 0;
@@ -259,6 +261,19 @@ struct mf_ctx {
 
 namespace mf {
 
+// While it lives, boundary passes take the time t by value instead of
+// reading the step's time from device memory (which captured steps need).
+struct HostTime {
+    mf_ctx* c;
+    HostTime(mf_ctx* ctx, double t) : c(ctx)
+    {
+        c->host_time = true;
+        c->t_host = t;
+    }
+    void set(double t) { c->t_host = t; }
+    ~HostTime() { c->host_time = false; }
+};
+
 constexpr int kGraphSteps = 16;  // SSPRK33 steps per multi-step graph
 
 // error helpers
@@ -335,13 +350,19 @@ struct StageOut {
     double dt = 0.0;
     const double* uprev = nullptr;
     double* out = nullptr;
-    // stepping with the residual viscosity: sums_out applies the next
-    // rhs!'s first boundary pass (at (t + out_t_adv) + out_dt_off) to the
-    // output and leaves the output's per-block sums in d_stage_psum;
-    // sums_in: this rhs!'s input came so (its first pass and sum pass are
-    // skipped)
-    bool sums_out = false, sums_in = false;
-    double out_t_adv = 0.0, out_dt_off = 0.0;
+    // stepping: handed_out applies the next rhs!'s first boundary pass (at
+    // the step's time, or t_next with out_t_next, + out_dt_off) to the
+    // output, with the residual viscosity also leaves the output's per-block
+    // sums in d_stage_psum, and with keep_raw the boundary entries' values
+    // before the pass in d_sraw; handed_in: this rhs!'s input came so (its
+    // first pass and sum pass are skipped)
+    bool handed_out = false, handed_in = false, keep_raw = false;
+    bool out_t_next = false;
+    double out_dt_off = 0.0;
+    // what the kernel that writes the output does to the step's time
+    enum { kTimeKeep = 0, kTimeNext, kTimeAdvance };
+    int time = kTimeKeep;
+    bool u_dead = false;  // the input is not read again: no second boundary pass on it
 };
 int run_rhs(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off, const StageOut& st);
 // parts of one rhs! (for timing single kernels)
@@ -352,8 +373,12 @@ int run_set_time(mf_ctx* c, double t, int success_iter);
 // History callback; with advance_dt != 0 it first ends the step (t += dt,
 // success_iter += 1) in the same launch.
 int run_history(mf_ctx* c, const double* d_u, int init, double advance_dt = 0.0);
-int run_advance_time(mf_ctx* c, double dt);
+// the boundary entries' raw values (d_sraw) back into d_u
+int run_restore_raw(mf_ctx* c, double* d_u);
 int run_limiter(mf_ctx* c, double* d_u, double thr, int var);
+// the first boundary pass (at the step's time + dt_off) and its transpose
+int bc_pass_state(mf_ctx* c, double* d_u, double dt_off);
+int bc_pass_homog(mf_ctx* c, double* d_u);
 int run_axpby(mf_ctx* c, int64_t n, double a, const double* x, double b, double* y);
 int run_fill(mf_ctx* c, double* p, int64_t n, double v);
 

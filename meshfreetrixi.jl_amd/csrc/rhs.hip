@@ -34,7 +34,6 @@ __device__ __forceinline__ void slip_project(const double* nrm2, double* s)
 struct BcArgs {
     int e0, e1;
     const int32_t* bidx;
-    const int32_t* btag;
     const double* bnormal;
     const double* btable;
     const double* px;
@@ -42,59 +41,29 @@ struct BcArgs {
     const uint8_t* flag;   // per node (fused use)
     const int32_t* entry;  // per node (fused use)
     double gamma;
-    const StepScalars* sc;
+    const double* tp;  // the pass's time is *tp + dt_off (captured steps), or
+    double t0;         // t0 + dt_off with tp null (the time by value)
     double dt_off;
-    double t_adv;  // the pass's time is (sc->t + t_adv) + dt_off (t_adv = 0: sc->t + dt_off)
     int homog;
-    const int32_t* tag_kind;  // per tag, device tables
-    const int32_t* tag_fn;
-    const double* tag_params;  // 8 per tag
+    int slip_only;             // the second pass: slip walls only
+    const double* tag_params;  // 8 per tag, device table
     const int32_t* ecode;      // per entry: first-pass kind | function << 4 | tag << 8
 };
 
 // The first-pass condition of boundary entry e on the state s of its node;
-// false if the entry leaves the state unchanged.
-template <int V>
-__device__ __forceinline__ bool bc_entry(const BcArgs& b, int e, int32_t node, double* s)
-{
-    const int tag = b.btag[e];
-    const int kind = b.tag_kind[tag];
-    if (kind == MF_BC_DIRICHLET) {
-        if (b.homog) {
-#pragma unroll
-            for (int v = 0; v < V; ++v) s[v] = 0.0;
-        } else if (b.tag_fn[tag] == MF_FN_TABLE) {
-#pragma unroll
-            for (int v = 0; v < V; ++v) s[v] = b.btable[(int64_t)e * V + v];
-        } else {
-            double t = b.sc->t;
-            if (b.t_adv != 0.0) t = t + b.t_adv;
-            t = t + b.dt_off;
-            bc_value<V>(b.tag_fn[tag], b.tag_params + 8 * tag, b.gamma, b.px[node], b.py[node], t, s);
-        }
-        return true;
-    }
-    if (kind == MF_BC_SLIP_WALL) {
-        if constexpr (V == 4) {
-            slip_project(b.bnormal + 2 * e, s);
-            return true;
-        }
-    }
-    return false;
-}
-
-// bc_entry's first pass for node `node` with boundary entry e, from the
-// entry's packed code: the code, the node's coordinates and the time load
-// together, then the tag's parameters (or the entry's table row or normal):
-// two dependent loads after the entry index instead of bc_entry's four;
-// same arithmetic.
+// false if the entry leaves the state unchanged.  From the entry's packed
+// code: the code, the node's coordinates and the time load together, then
+// the tag's parameters (or the entry's table row or normal): two dependent
+// loads after the entry index, where the tag, its kind, its function and its
+// parameters one after another were four.
 template <int V>
 __device__ __forceinline__ bool bc_node(const BcArgs& b, int e, int32_t node, double* s)
 {
     const int32_t code = b.ecode[e];
-    const double xn = b.px[node], yn = b.py[node], t0 = b.sc->t;
+    const double xn = b.px[node], yn = b.py[node], t0 = b.tp ? *b.tp : b.t0;
     const int kind = code & 15, fn = (code >> 4) & 15, tag = code >> 8;
     if (kind == MF_BC_DIRICHLET) {
+        if (b.slip_only) return false;
         if (b.homog) {
 #pragma unroll
             for (int v = 0; v < V; ++v) s[v] = 0.0;
@@ -102,10 +71,7 @@ __device__ __forceinline__ bool bc_node(const BcArgs& b, int e, int32_t node, do
 #pragma unroll
             for (int v = 0; v < V; ++v) s[v] = b.btable[(int64_t)e * V + v];
         } else {
-            double t = t0;
-            if (b.t_adv != 0.0) t = t + b.t_adv;
-            t = t + b.dt_off;
-            bc_value<V>(fn, b.tag_params + 8 * tag, b.gamma, xn, yn, t, s);
+            bc_value<V>(fn, b.tag_params + 8 * tag, b.gamma, xn, yn, t0 + b.dt_off, s);
         }
         return true;
     }
@@ -195,14 +161,31 @@ struct RhsArgs {
     double dt;
     const double* __restrict__ uprev;
     double* __restrict__ out;
-    // stepping: the output is the next rhs!'s input.  With stage_psum set
-    // the transposed kernel applies that rhs!'s first boundary pass (obc)
-    // to the output and stores the output's per-block sums there (tile or
-    // node block t at 4 t), which that rhs!'s max pass reads in place of
-    // its own sum pass
+    // stepping: the output is the next rhs!'s input.  With obc.flag set the
+    // kernel that writes the output applies that rhs!'s first boundary pass
+    // (obc) to it; sraw, if set, keeps the values before it (one state per
+    // boundary entry).  With stage_psum set the transposed kernel also stores
+    // the output's per-block sums there (tile or node block t at 4 t), which
+    // that rhs!'s max pass reads in place of its own sum pass.
     double* __restrict__ stage_psum;
     BcArgs obc;
+    double* __restrict__ sraw;
+    // stepping: the kernel that writes the output also moves the step's time
+    // on (tm_dst, if set, = *tm_src + tm_add; *tm_iter += 1), between device
+    // variables that nothing else in the launch touches
+    double* tm_dst;
+    const double* tm_src;
+    double tm_add;
+    int* tm_iter;
 };
+
+__device__ __forceinline__ void move_time(const RhsArgs& a)
+{
+    if (a.tm_dst && blockIdx.x == 0 && threadIdx.x == 0) {
+        *a.tm_dst = *a.tm_src + a.tm_add;
+        if (a.tm_iter) *a.tm_iter = *a.tm_iter + 1;
+    }
+}
 
 // FP32 node records (split-FP32 intermediates): V floats per record.
 template <int V>
@@ -281,29 +264,31 @@ __device__ __forceinline__ void stage_value(const RhsArgs& a, int64_t i, const d
     }
 }
 
+// The output of node i: du, or the next stage with, in stepping, the first
+// boundary pass of the rhs! that reads it; o returns the stored stage.
 template <int V>
-__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* du)
+__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* du, double* o)
 {
     if (a.st_kind == ST_NONE) {
         store_state<V>(a.du, i, du);
         return;
     }
-    double o[V];
     stage_value<V>(a, i, du, o);
+    if (a.obc.flag) {
+        const int32_t e = a.obc.entry[i];
+        if (e >= 0) {
+            if (a.sraw) store_state<V>(a.sraw, e, o);
+            bc_node<V>(a.obc, e, (int32_t)i, o);
+        }
+    }
     store_state<V>(a.out, i, o);
 }
 
-// emit() of a stage whose output the next rhs! reads (a.stage_psum set):
-// that rhs!'s first boundary pass is applied to the output here, as its
-// sum pass would apply it, and o returns the stored state for the sums.
-__device__ __forceinline__ void emit_staged(const RhsArgs& a, int64_t i, const double* du, double* o)
+template <int V>
+__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* du)
 {
-    stage_value<4>(a, i, du, o);
-    if (a.obc.flag) {
-        const int32_t e = a.obc.entry[i];
-        if (e >= 0) bc_node<4>(a.obc, e, (int32_t)i, o);
-    }
-    store_state<4>(a.out, i, o);
+    double o[V];
+    emit<V>(a, i, du, o);
 }
 
 // Residual/upwind viscosity at node i (hyperviscosity.jl:246-349): eps_uw
@@ -566,6 +551,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int64_t N = a.N;
@@ -772,6 +758,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int K = NS ? NS : a.k;
@@ -844,6 +831,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
+    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int64_t N = a.N;
@@ -1011,6 +999,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
     constexpr int RU = (HG ? 2 : 0) + (HL ? 1 : 0);  // V-value units per halo record
     constexpr int LU = HG ? 2 : 0;                   // unit of L in a record
     extern __shared__ double lds[];
+    move_time(a);
     int64_t i, off = 0;
     int W = 0;
     const int lane = threadIdx.x & 63;
@@ -1211,14 +1200,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             }
         }
         mask_du<V>(a, i, du);
-        if constexpr (V == 4) {
-            if (a.stage_psum)
-                emit_staged(a, i, du, o);
-            else
-                emit<V>(a, i, du);
-        } else {
-            emit<V>(a, i, du);
-        }
+        emit<V>(a, i, du, o);
     }
     if constexpr (V == 4) {
         if (a.stage_psum) {  // the same for the whole block
@@ -1243,7 +1225,18 @@ __global__ __launch_bounds__(kBlock) void k_bc_state(const BcArgs b, double* u)
     const int32_t node = b.bidx[e];
     double s[V];
     load_state<V>(u, node, s);
-    if (bc_entry<V>(b, e, node, s)) store_state<V>(u, node, s);
+    if (bc_node<V>(b, e, node, s)) store_state<V>(u, node, s);
+}
+
+// The values of boundary entries before the first boundary pass back into u.
+template <int V>
+__global__ __launch_bounds__(kBlock) void k_bc_restore(int nb, const int32_t* bidx, const double* sraw, double* u)
+{
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= nb) return;
+    double s[V];
+    load_state<V>(sraw, e, s);
+    store_state<V>(u, bidx[e], s);
 }
 
 // ------------------------------------ residual-viscosity reductions
@@ -1345,22 +1338,14 @@ __global__ void k_set_time(StepScalars* sc, double t, int success_iter, int set_
     }
 }
 
-__global__ void k_advance_time(StepScalars* sc, double dt)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        sc->t = sc->t + dt;
-        sc->success_iter = sc->success_iter + 1;
-    }
-}
-
 // HistoryCallback (history.jl:91-152).  Single thread: shift the time
 // history, count the points in use and solve the transposed Vandermonde
 // system for the derivative weights (partial-pivoting LU, as `A' \ b`).
 // One thread.  The step scalars are read once into registers, the
 // shifted history and the weights are computed there, and the results are
 // stored once: every global access in a dependent chain would cost a
-// memory round trip.  With `advance` set it first ends the step as
-// k_advance_time does (t += dt, success_iter += 1), saving that launch.
+// memory round trip.  With `advance` set it first ends the step (t += dt,
+// success_iter += 1).
 __global__ __launch_bounds__(64) void k_history_weights(StepScalars* sc, int P, int init, int advance, double dt)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -1993,6 +1978,7 @@ __global__ __launch_bounds__(kBlock) void k_igr_x(const IgrArgs a, int it)
 template <int BT>
 __global__ __launch_bounds__(kBlock) void k_igr_apply(const IgrArgs g, const RhsArgs a)
 {
+    move_time(a);
     const int64_t i = remapped_node();
     if (i >= g.N) return;
     const double2 s = igr_grad<BT>(g, i, g.x);
@@ -2131,19 +2117,17 @@ static BcArgs make_bc(mf_ctx* c, double dt_off, int homog)
 {
     BcArgs b{};
     b.bidx = c->bc.bidx;
-    b.btag = c->bc.btag;
     b.bnormal = c->bc.bnormal;
     b.btable = c->bc.btable;
     b.px = c->d_x;
     b.py = c->d_y;
     b.gamma = c->p0;
-    b.sc = c->d_sc;
+    b.tp = c->host_time ? nullptr : &c->d_sc->t;
+    b.t0 = c->t_host;
     b.flag = c->bc.flag;
     b.entry = c->bc.entry;
     b.dt_off = dt_off;
     b.homog = homog;
-    b.tag_kind = c->bc.d_kind;
-    b.tag_fn = c->bc.d_fn;
     b.tag_params = c->bc.d_params;
     b.ecode = c->bc.ecode;
     return b;
@@ -2173,7 +2157,7 @@ static int bc_state_pass(mf_ctx* c, double* u, double dt_off, int homog, bool sl
     if (!c->have_bc || c->bc.nb == 0) return MF_OK;
     if (slip_only && !c->bc.any_slip) return MF_OK;
     BcArgs b = make_bc(c, dt_off, homog);
-    if (slip_only) b.tag_kind = c->bc.d_kind_slip;
+    b.slip_only = slip_only ? 1 : 0;
     auto launch = [&](int e0, int e1) {
         if (e1 <= e0) return;
         b.e0 = e0;
@@ -2432,12 +2416,13 @@ int run_rhs_parts(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off,
     // a stage handed over by the previous rhs! (stepping) has had this
     // rhs!'s first boundary pass and carries its sums
     const int64_t nblk = (c->N + kBlock - 1) / kBlock;
-    if (st.sums_in || st.sums_out) {
-        if (c->visc_mode != MF_VISC_RESIDUAL || igr || !c->d_stage_psum || (c->have_bc && c->bc.multi) ||
-            (c->tiles_b && c->n_tiles != nblk))
-            return fail(c, MF_ERR_STATE, "rhs!: stage sums without the residual viscosity's transposed kernel");
+    const bool residual = c->visc_mode == MF_VISC_RESIDUAL;
+    if (st.handed_in || st.handed_out) {
+        if (igr || (c->have_bc && c->bc.multi) ||
+            (residual && (!c->d_stage_psum || (c->tiles_b && c->n_tiles != nblk))))
+            return fail(c, MF_ERR_STATE, "rhs!: a stage cannot be handed over with these sources and boundaries");
     }
-    int rc = ((parts & RHS_BC) && !fused_bc && !st.sums_in) ? bc_state_pass(c, d_u, dt_off, 0, false) : MF_OK;
+    int rc = ((parts & RHS_BC) && !fused_bc && !st.handed_in) ? bc_state_pass(c, d_u, dt_off, 0, false) : MF_OK;
     if (rc) return rc;
     // with the IGR source the other kernels leave du (masked) for its last
     // kernel, which writes the output
@@ -2446,19 +2431,33 @@ int run_rhs_parts(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off,
     out_args.dt = st.dt;
     out_args.uprev = st.uprev;
     out_args.out = st.out;
-    if (st.sums_out) {
-        out_args.stage_psum = c->d_stage_psum;
-        out_args.obc = make_bc(c, st.out_dt_off, 0);
-        out_args.obc.t_adv = st.out_t_adv;
-        if (!c->have_bc) out_args.obc.flag = nullptr;
+    if (st.handed_out) {
+        if (residual) out_args.stage_psum = c->d_stage_psum;
+        if (c->have_bc) {
+            out_args.obc = make_bc(c, st.out_dt_off, 0);
+            if (st.out_t_next) out_args.obc.tp = &c->d_sc->t_next;
+            out_args.sraw = st.keep_raw ? c->d_sraw : nullptr;
+        }
+    }
+    if (st.time == StageOut::kTimeNext) {  // t_next = t + dt
+        out_args.tm_dst = &c->d_sc->t_next;
+        out_args.tm_src = &c->d_sc->t;
+        out_args.tm_add = st.dt;
+    } else if (st.time == StageOut::kTimeAdvance) {  // t = t_next, one more step
+        out_args.tm_dst = &c->d_sc->t;
+        out_args.tm_src = &c->d_sc->t_next;
+        out_args.tm_iter = &c->d_sc->success_iter;
     }
     RhsArgs a = out_args;
-    if (igr) a.st_kind = ST_NONE;
+    if (igr) {
+        a.st_kind = ST_NONE;
+        a.tm_dst = nullptr;
+    }
     const unsigned grid = xcd_grid(nblk);
     if (rv || tom) {
         if (rv && c->visc_mode == MF_VISC_RESIDUAL && (parts & RHS_REDUCE)) {
             const int ns = c->n_psum, nm = c->n_pmax;
-            if (st.sums_in) {
+            if (st.handed_in) {
                 launch_k(c, 3, k_rv_max, dim3(nm), dim3(kBlock), 0, c->N, (c->N + nm - 1) / nm, (const double*)d_u,
                          (const double*)c->d_stage_psum, (int)nblk, c->d_partials + 4 * ns, c->d_sc);
             } else {
@@ -2473,6 +2472,7 @@ int run_rhs_parts(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off,
         RhsArgs pa = a;
         pa.st_kind = ST_NONE;
         pa.stage_psum = nullptr;
+        pa.tm_dst = nullptr;
         if (parts & RHS_FLUX) launch_flux_v<4>(c, prec, pa, hvk, rv, grid);
         if (parts & RHS_TRANSPOSE) {
             const int gt = (rv ? 1 : 0) | (tom ? 2 : 0);
@@ -2494,7 +2494,8 @@ int run_rhs_parts(mf_ctx* c, int prec, double* d_u, double* d_du, double dt_off,
     MF_HIP(c, hipGetLastError());
     if (igr && (parts & RHS_IGR) && (rc = run_igr(c, d_u, out_args, grid))) return rc;
     // second boundary pass on u: only the slip projection changes anything
-    rc = (parts & RHS_BC) ? bc_state_pass(c, d_u, dt_off, 0, true) : MF_OK;
+    // (not where the caller reads u no more)
+    rc = (parts & RHS_BC) && !st.u_dead ? bc_state_pass(c, d_u, dt_off, 0, true) : MF_OK;
     return rc;
 }
 
@@ -2506,9 +2507,14 @@ int run_set_time(mf_ctx* c, double t, int success_iter)
     return MF_OK;
 }
 
-int run_advance_time(mf_ctx* c, double dt)
+int run_restore_raw(mf_ctx* c, double* d_u)
 {
-    hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(1), 0, c->stream, c->d_sc, dt);
+    const unsigned g = (unsigned)((c->bc.nb + kBlock - 1) / kBlock);
+    if (g == 0) return MF_OK;
+    if (c->nvar == 4)
+        hipLaunchKernelGGL(k_bc_restore<4>, dim3(g), dim3(kBlock), 0, c->stream, c->bc.nb, c->bc.bidx, c->d_sraw, d_u);
+    else
+        hipLaunchKernelGGL(k_bc_restore<1>, dim3(g), dim3(kBlock), 0, c->stream, c->bc.nb, c->bc.bidx, c->d_sraw, d_u);
     MF_HIP(c, hipGetLastError());
     return MF_OK;
 }
