@@ -280,11 +280,7 @@ static int upload_fields(mf_ctx* c, double* d_dst, const double* const* fields)
     if (!fields) return fail(c, MF_ERR_ARGUMENT, "null fields");
     for (int v = 0; v < c->nvar; ++v)
         if (!fields[v]) return fail(c, MF_ERR_ARGUMENT, "null field pointer");
-    // stage in d_T (SoA), then interleave
-    for (int v = 0; v < c->nvar; ++v)
-        MF_HIP(c, hipMemcpyAsync(c->d_T + (size_t)v * c->N, fields[v], sizeof(double) * c->N,
-                                 hipMemcpyHostToDevice, c->stream));
-    return launch_soa_to_aos(c, c->d_T, d_dst);
+    return upload_state(c, d_dst, fields);
 }
 
 static int download_fields(mf_ctx* c, const double* d_src, double* const* fields)
@@ -292,13 +288,7 @@ static int download_fields(mf_ctx* c, const double* d_src, double* const* fields
     if (!fields) return fail(c, MF_ERR_ARGUMENT, "null fields");
     for (int v = 0; v < c->nvar; ++v)
         if (!fields[v]) return fail(c, MF_ERR_ARGUMENT, "null field pointer");
-    int rc = launch_aos_to_soa(c, d_src, c->d_T);
-    if (rc) return rc;
-    for (int v = 0; v < c->nvar; ++v)
-        MF_HIP(c, hipMemcpyAsync(fields[v], c->d_T + (size_t)v * c->N, sizeof(double) * c->N,
-                                 hipMemcpyDeviceToHost, c->stream));
-    MF_HIP(c, hipStreamSynchronize(c->stream));
-    return MF_OK;
+    return download_state(c, d_src, fields);
 }
 
 }  // namespace mf
@@ -327,6 +317,7 @@ int mf_ctx_create(int device, mf_ctx** out)
         delete c;
         return MF_ERR_HIP;
     }
+    pinned_pool_open();
     *out = c;
     return MF_OK;
 }
@@ -353,6 +344,7 @@ int mf_ctx_destroy(mf_ctx* c)
     dfree(c->d_flush);
     (void)hipStreamDestroy(c->stream);
     delete c;
+    pinned_pool_close();
     return MF_OK;
 }
 
@@ -483,17 +475,17 @@ int mf_knn(mf_ctx* c, int k, int32_t* idx_out, double* dist_out, double* dx_min,
         int32_t* rows = nullptr;
         if ((rc = dalloc(c, &rows, (size_t)k * c->N))) return rc;
         if ((rc = launch_ell_to_rows(c, c->d_idx, rows, k))) return rc;
-        MF_HIP(c, hipMemcpyAsync(idx_out, rows, sizeof(int32_t) * k * c->N, hipMemcpyDeviceToHost, c->stream));
-        MF_HIP(c, hipStreamSynchronize(c->stream));
+        rc = copy_array(c, rows, idx_out, sizeof(int32_t) * k * c->N, true);
         dfree(rows);
+        if (rc) return rc;
     }
     if (dist_out) {
         double* rows = nullptr;
         if ((rc = dalloc(c, &rows, (size_t)k * c->N))) return rc;
         if ((rc = launch_ell_to_rows_d(c, d2, rows, k))) return rc;
-        MF_HIP(c, hipMemcpyAsync(dist_out, rows, sizeof(double) * k * c->N, hipMemcpyDeviceToHost, c->stream));
-        MF_HIP(c, hipStreamSynchronize(c->stream));
+        rc = copy_array(c, rows, dist_out, sizeof(double) * k * c->N, true);
         dfree(rows);
+        if (rc) return rc;
         for (int64_t q = 0; q < (int64_t)k * c->N; ++q) dist_out[q] = std::sqrt(dist_out[q]);
     }
     MF_HIP(c, hipStreamSynchronize(c->stream));
@@ -535,7 +527,10 @@ int mf_set_stencil(mf_ctx* c, const int32_t* idx, int64_t n_points, int k)
     if ((rc = set_k(c, k))) return rc;
     int32_t* rows = nullptr;
     if ((rc = dalloc(c, &rows, (size_t)k * c->N))) return rc;
-    MF_HIP(c, hipMemcpyAsync(rows, idx, sizeof(int32_t) * k * c->N, hipMemcpyHostToDevice, c->stream));
+    if ((rc = copy_array(c, rows, idx, sizeof(int32_t) * k * c->N, false))) {
+        dfree(rows);
+        return rc;
+    }
     if ((rc = launch_rows_to_ell(c, rows, c->d_idx, k))) return rc;
     if ((rc = stencil_ready(c))) return rc;
     MF_HIP(c, hipStreamSynchronize(c->stream));
@@ -638,8 +633,7 @@ int mf_compute_operator(mf_ctx* c, int phs_power, int poly_degree, int deriv_ord
             if (!out) continue;
             if (!rows && (r = dalloc(c, &rows, n))) return r;
             if ((r = launch_ell_to_rows_d(c, w == 0 ? wx : wy, rows, c->k))) return r;
-            MF_HIP(c, hipMemcpyAsync(out, rows, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
-            MF_HIP(c, hipStreamSynchronize(c->stream));
+            if ((r = copy_array(c, rows, out, sizeof(double) * n, true))) return r;
         }
         MF_HIP(c, hipStreamSynchronize(c->stream));
         return MF_OK;
@@ -671,11 +665,11 @@ int mf_set_operator(mf_ctx* c, int target, const double* wx, const double* wy)
         int r;
         if ((r = dalloc(c, &rx, n)) || (r = dalloc(c, &ex, n))) return r;
         if (wy && (r = dalloc(c, &ey, n))) return r;
-        MF_HIP(c, hipMemcpyAsync(rx, wx, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+        if ((r = copy_array(c, rx, wx, sizeof(double) * n, false))) return r;
         if ((r = launch_rows_to_ell_d(c, rx, ex, c->k))) return r;
         if (wy) {
             MF_HIP(c, hipStreamSynchronize(c->stream));
-            MF_HIP(c, hipMemcpyAsync(rx, wy, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+            if ((r = copy_array(c, rx, wy, sizeof(double) * n, false))) return r;
             if ((r = launch_rows_to_ell_d(c, rx, ey, c->k))) return r;
         }
         if ((r = alloc_op(c, target))) return r;
@@ -810,9 +804,16 @@ int mf_weights_ragged_get(mf_ctx* c, double* wx, double* wy)
     if (c->rn == 0) return fail(c, MF_ERR_STATE, "mf_weights_ragged_get: no stencils");
     int st = 0;
     MF_HIP(c, hipMemcpyAsync(&st, c->d_status, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    if (wx) MF_HIP(c, hipMemcpyAsync(wx, c->d_rwx, sizeof(double) * c->rnnz, hipMemcpyDeviceToHost, c->stream));
-    if (wy) MF_HIP(c, hipMemcpyAsync(wy, c->d_rwy, sizeof(double) * c->rnnz, hipMemcpyDeviceToHost, c->stream));
+    int rc2 = MF_OK;
+    for (int w = 0; w < 2 && rc2 == MF_OK; ++w) {
+        HostFields f;
+        f.count = 1;
+        f.field_bytes = sizeof(double) * (size_t)c->rnnz;
+        f.fields[0] = w == 0 ? wx : wy;
+        if (f.fields[0]) rc2 = copy_fields(c, w == 0 ? c->d_rwx : c->d_rwy, f, true);
+    }
     MF_HIP(c, hipStreamSynchronize(c->stream));
+    if (rc2) return rc2;
     if (st) return fail(c, MF_ERR_SINGULAR, "ragged weights: singular stencil system");
     return MF_OK;
 }
@@ -1214,6 +1215,21 @@ int mf_rhs_host(mf_ctx* c, double t, int precision, double* const* u, double* co
     int rc = check_ctx(c);
     if (rc) return rc;
     if ((rc = prepare_rhs(c))) return rc;
+    if (!u || !du) return fail(c, MF_ERR_ARGUMENT, "null fields");
+    for (int v = 0; v < c->nvar; ++v)
+        if (!u[v] || !du[v]) return fail(c, MF_ERR_ARGUMENT, "null field pointer");
+    {
+        const HostTime time(c, t);
+        bool done;
+        rc = rhs_through_pinned(
+            c, c->d_buf[MF_BUF_U], c->d_buf[MF_BUF_DU], u, du,
+            [&]() -> int {
+                c->fsal_valid = false;
+                return run_rhs(c, precision, c->d_buf[MF_BUF_U], c->d_buf[MF_BUF_DU], 0.0, StageOut());
+            },
+            &done);
+        if (rc || done) return rc;
+    }
     if ((rc = upload_fields(c, c->d_buf[MF_BUF_U], u))) return rc;
     if ((rc = mf_rhs(c, t, precision))) return rc;
     if ((rc = download_fields(c, c->d_buf[MF_BUF_DU], du))) return rc;

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -288,6 +289,25 @@ int hip_fail(mf_ctx* c, hipError_t e, const char* what);
 template <class T>
 int dalloc(mf_ctx* c, T** p, size_t count);
 void dfree(void* p);
+
+// ------------------------------------------------ host_copy.hip
+// a contiguous device range as `count` host fields of field_bytes each
+struct HostFields {
+    int count = 0;
+    size_t field_bytes = 0;
+    void* fields[kMaxVar] = {nullptr, nullptr, nullptr, nullptr};
+};
+// the pool of pinned chunks lives as long as some context is open
+void pinned_pool_open();
+void pinned_pool_close();
+int copy_fields(mf_ctx* c, void* d, const HostFields& f, bool to_host);
+int copy_array(mf_ctx* c, void* d, const void* h, size_t bytes, bool to_host);
+// a state (node-major on the device) from / to the caller's fields; the
+// caller's arrays are read or complete on return
+int upload_state(mf_ctx* c, double* d_dst, const double* const* fields);
+int download_state(mf_ctx* c, const double* d_src, double* const* fields);
+int rhs_through_pinned(mf_ctx* c, double* d_u, double* d_du, double* const* u, double* const* du,
+                       const std::function<int()>& run, bool* done);
 
 // XCD-aware launch helper: blocks are dealt round-robin to the 8 XCDs; the
 // remap gives every XCD one contiguous range of logical blocks.

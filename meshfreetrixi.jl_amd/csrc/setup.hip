@@ -1405,12 +1405,13 @@ int launch_rows_to_ell_d(mf_ctx* c, const double* d_rows, double* d_ell, int k)
     return MF_OK;
 }
 
-__global__ void k_soa_to_aos(int64_t N, int V, const double* soa, double* aos, const int32_t* uid)
+// Both read and write the fields in order, also where they are host memory.
+__global__ void k_soa_to_aos(int64_t N, int V, const double* soa, double* aos, const int32_t* inv)
 {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= N * V) return;
-    const int64_t p = q / V, v = q % V;
-    aos[q] = soa[v * N + uid[p]];
+    const int64_t v = q / N, u = q % N;
+    aos[(int64_t)inv[u] * V + v] = soa[q];
 }
 
 __global__ void k_aos_to_soa(int64_t N, int V, const double* aos, double* soa, const int32_t* inv)
@@ -1425,7 +1426,7 @@ int launch_soa_to_aos(mf_ctx* c, const double* d_soa, double* d_aos)
 {
     const int64_t n = c->N * c->nvar;
     hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, c->N,
-                       c->nvar, d_soa, d_aos, c->d_uid);
+                       c->nvar, d_soa, d_aos, c->d_inv);
     MF_HIP(c, hipGetLastError());
     return MF_OK;
 }

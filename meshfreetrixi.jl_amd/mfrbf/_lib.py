@@ -278,6 +278,14 @@ class Context:
         self._chk(self._L.mf_state_download(self.h, buf, self._fields(out)))
         return out
 
+    def download_rows(self, buf, out):
+        """download into a float64 (nvar, N) array whose rows are contiguous,
+        such as a column range of a larger array."""
+        assert out.dtype == np.float64 and out.shape == (self.nvar, self.N) and out.strides[1] == 8, \
+            "the rows must be contiguous float64 of length N"
+        self._chk(self._L.mf_state_download(self.h, buf, fields_ptr(out)))
+        return out
+
     def rhs(self, t, precision=MF_PREC_F64):
         self._chk(self._L.mf_rhs(self.h, t, precision))
 

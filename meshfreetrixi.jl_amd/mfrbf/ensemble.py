@@ -150,4 +150,9 @@ class EnsembleLanes:
 
     def download(self):
         """The ensemble's state (nvar, N), clouds in the order of `specs`."""
-        return np.concatenate([lane.ctx.download(L.MF_BUF_U) for lane in self.lanes], axis=1)
+        out = np.empty((4, self.N))
+        at = 0
+        for lane in self.lanes:  # each lane's fields straight into their place
+            lane.ctx.download_rows(L.MF_BUF_U, out[:, at:at + lane.N])
+            at += lane.N
+        return out
