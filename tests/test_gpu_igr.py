@@ -12,6 +12,7 @@ import oracle as O
 from conftest import rel_inf
 from mfrbf import _lib as L
 from mfrbf import configs
+from mfrbf.clouds import cloud_square
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +114,32 @@ def test_ssprk33_igr(mf):
         c.ctx.upload(L.MF_BUF_U, c.u0.copy())
         c.ctx.ssprk33(0.0, c.dt, 4, flags=flags)
         assert rel_inf(c.ctx.download(L.MF_BUF_U), uo) < 1e-10, flags
+
+
+@pytest.mark.parametrize("side,k", [(4, 3), (8, 5), (16, 6), (17, 11), (33, 30), (40, 31)])
+def test_igr_tiles_at_the_edges(side, k):
+    """Batches and halos of every remainder (one tile and several, K below, at
+    and above the batch and twice the batch): sigma and du over the LDS tiles
+    are the bits of the global gathers, and du the same on a second call."""
+    _say("igr tiles side=%d k=%d" % (side, k))
+    rng = np.random.default_rng(100 * side + k)
+    x, y, _, _, _ = cloud_square(side, side)
+    n = len(x)
+    ctx = L.Context(0)
+    ctx.set_equations(L.MF_EQ_EULER_2D, 1.4)
+    ctx.set_points(x, y)
+    ctx.set_stencil(ctx.knn(k)[0])
+    ctx.set_operator(L.MF_OP_FLUX, rng.standard_normal((n, k)), rng.standard_normal((n, k)))
+    ctx.set_source_igr(1e-4, 20)
+    u0 = np.ascontiguousarray(np.stack([1.0 + 0.1 * rng.random(n), 0.1 * rng.standard_normal(n),
+                                        0.1 * rng.standard_normal(n), 5.0 + rng.random(n)]))
+    out = []
+    for tiles in (1, 1, 0):
+        ctx.set_tuning(L.MF_TUNE_TILES, tiles)
+        du = np.empty_like(u0)
+        ctx.rhs_host(0.0, u0.copy(), du, L.MF_PREC_F64)
+        assert ctx.tile_info()["tiles_a"] == tiles
+        out.append((du, ctx.igr_sigma()))
+    assert np.isfinite(out[0][0]).all() and np.abs(out[0][1]).max() > 0.0
+    for du, sigma in out[1:]:
+        assert np.array_equal(du, out[0][0]) and np.array_equal(sigma, out[0][1])
