@@ -1082,7 +1082,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             const int64_t slice = i >> 6;
             off = a.sell_off[slice];
             W = a.sell_w[slice];
-            load(0, q0);
+            if (W > 0) load(0, q0);  // a slice of nodes that no stencil names has no entries
         }
     }
     double tx[V], ty[V], th[V];

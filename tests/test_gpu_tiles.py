@@ -138,3 +138,24 @@ def test_advection_tiles_and_vjp():
         if tiles:
             assert ctx.tile_info()["tiles_a"] and ctx.tile_info()["tiles_b"]
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("n,unnamed", [(1000, 64), (1000, 300), (1024, 1), (1024, 600), (129, 65)])
+def test_slices_that_no_stencil_names(n, unnamed):
+    """The last nodes, and 64 in the middle, are in no stencil: their slices of
+    the transposed operator have no entries (a whole tile of them with 300 and
+    600), and the kernels load none."""
+    rng = np.random.default_rng(n + unnamed)
+    k = 12
+    ctx = L.Context(0)
+    ctx.set_equations(L.MF_EQ_EULER_2D, 1.4)
+    ctx.set_points(rng.random(n), rng.random(n))
+    ctx.set_stencil(np.tile(np.arange(k, dtype=np.int32), (n, 1)))
+    order = ctx.node_order()
+    named = np.setdiff1d(np.arange(n - unnamed), np.arange(64, 128) if n > 200 else [])
+    row = np.minimum(np.arange(n), len(named) - k)
+    idx = np.empty((n, k), np.int32)
+    idx[order] = order[named[row[:, None] + np.arange(k)]]
+    operators(ctx, idx, rng)
+    both_ways(ctx, n, rng)
+    assert ctx.tile_info()["tiles_a"] == 0  # the last pass was the one without
