@@ -44,13 +44,11 @@ struct VjpArgs {
     const double2* twb;
 };
 
-// M^T lam at node r (the second boundary pass is its own transpose):
-// Dirichlet rows vanish, slip nodes drop the momentum.
+// M^T lam of a node with boundary flag f (the second boundary pass is its own
+// transpose): Dirichlet rows vanish, slip nodes drop the momentum.
 template <int V>
-__device__ __forceinline__ void mask_lam(const VjpArgs& a, int64_t r, double* l)
+__device__ __forceinline__ void mask_lam(uint32_t f, double* l)
 {
-    if (!a.flag) return;
-    const uint8_t f = a.flag[r];
     if (f & 1u)
 #pragma unroll
         for (int v = 0; v < V; ++v) l[v] = 0.0;
@@ -83,10 +81,28 @@ __device__ __forceinline__ void euler_jt(double gamma, const double* u, const do
     o[3] = a13 * gx[1] + a33 * gx[3] + b23 * gy[2] + b33 * gy[3];
 }
 
+// What the epilogue reads of its node; the tiled kernel loads it ahead of the
+// row's entries.
+template <int V>
+struct VjpTail {
+    double x[V], add[3][V];
+    uint32_t flag;
+};
+
+template <int V>
+__device__ __forceinline__ void load_tail(const VjpArgs& a, int64_t i, VjpTail<V>& t)
+{
+    if constexpr (V == 4) load_state<V>(a.x, i, t.x);
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        if (a.add[q]) load_state<V>(a.add[q], i, t.add[q]);
+    t.flag = a.flag ? a.flag[i] : 0u;
+}
+
 // Epilogue of one node's product: scale, flux Jacobian transpose at the
 // (boundary-imposed) state, the added terms, then P^T.
 template <int V>
-__device__ __forceinline__ void vjp_finish(const VjpArgs& a, int64_t i, double* gx, double* gy)
+__device__ __forceinline__ void vjp_finish(const VjpArgs& a, int64_t i, const VjpTail<V>& t, double* gx, double* gy)
 {
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -97,35 +113,29 @@ __device__ __forceinline__ void vjp_finish(const VjpArgs& a, int64_t i, double* 
     if constexpr (V == 1) {
         o[0] = -(a.eq.a1 * gx[0] + a.eq.a2 * gy[0]);
     } else {
-        double ui[4], jt[4];
-        load_state<4>(a.x, i, ui);
-        euler_jt(a.eq.gamma, ui, gx, gy, jt);
+        double jt[4];
+        euler_jt(a.eq.gamma, t.x, gx, gy, jt);
 #pragma unroll
         for (int v = 0; v < 4; ++v) o[v] = -jt[v];
     }
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         if (!a.add[q]) continue;
-        double s[V];
-        load_state<V>(a.add[q], i, s);
 #pragma unroll
-        for (int v = 0; v < V; ++v) o[v] = fma(a.add_scale[q], s[v], o[v]);
+        for (int v = 0; v < V; ++v) o[v] = fma(a.add_scale[q], t.add[q][v], o[v]);
     }
     // P^T: Dirichlet rows vanish, slip nodes project the momentum
-    if (a.flag) {
-        const uint8_t f = a.flag[i];
-        if (f & 1u)
+    if (t.flag & 1u)
 #pragma unroll
-            for (int v = 0; v < V; ++v) o[v] = 0.0;
-        if constexpr (V == 4) {
-            if (f & 2u) {
-                const double* nr = a.bnormal + 2 * a.entry[i];
-                const double nn = sqrt(nr[0] * nr[0] + nr[1] * nr[1]);
-                const double e1 = nr[0] / nn, e2 = nr[1] / nn;
-                const double dot = o[1] * e1 + o[2] * e2;
-                o[1] -= dot * e1;
-                o[2] -= dot * e2;
-            }
+        for (int v = 0; v < V; ++v) o[v] = 0.0;
+    if constexpr (V == 4) {
+        if (t.flag & 2u) {
+            const double* nr = a.bnormal + 2 * a.entry[i];
+            const double nn = sqrt(nr[0] * nr[0] + nr[1] * nr[1]);
+            const double e1 = nr[0] / nn, e2 = nr[1] / nn;
+            const double dot = o[1] * e1 + o[2] * e2;
+            o[1] -= dot * e1;
+            o[2] -= dot * e2;
         }
     }
     store_state<V>(a.out, i, o);
@@ -149,21 +159,27 @@ __global__ __launch_bounds__(kBlock) void k_vjp(const VjpArgs a)
         const double2 w = a.tw[q];
         double l[V];
         load_state<V>(a.lam, r, l);
-        mask_lam<V>(a, r, l);
+        mask_lam<V>(a.flag ? a.flag[r] : 0u, l);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             gx[v] = fma(w.x, l[v], gx[v]);
             gy[v] = fma(w.y, l[v], gy[v]);
         }
     }
-    vjp_finish<V>(a, i, gx, gy);
+    VjpTail<V> tail;
+    load_tail<V>(a, i, tail);
+    vjp_finish<V>(a, i, tail, gx, gy);
 }
 
 // The same product over the LDS tiles of the transposed operator: the
 // tile's halo of M^T lam is staged once, the rows walk their entries in
-// batches of BT (every load of a batch issued first), in the same order as
-// k_vjp, so both give the same bits.
-template <int V, int BT>
+// batches of BT, two in turn, in the same order as k_vjp, so both give the
+// same bits.  At 65,536 nodes there is one tile per CU and the kernel is a
+// chain of waits for memory: the first batch and the node's own values are in
+// flight while the halo (two entries per thread and trip) is staged.
+// At that size, K = 30: 13.1 -> 11.2 us.  AHEAD: the node's values are held
+// through the sums.
+template <int V, int BT, bool AHEAD>
 __global__ __launch_bounds__(kBlock) void k_vjp_tl(const VjpArgs a)
 {
     extern __shared__ double lds[];
@@ -171,57 +187,77 @@ __global__ __launch_bounds__(kBlock) void k_vjp_tl(const VjpArgs a)
     if (t >= a.n_tiles) return;  // whole block
     const int64_t h0 = a.hb_off[t];
     const int nh = (int)(a.hb_off[t + 1] - h0);
-    for (int q = threadIdx.x; q < nh; q += kBlock) {
-        const int64_t r = a.hb_ids[h0 + q];
-        double l[V];
-        load_state<V>(a.lam, r, l);
-        mask_lam<V>(a, r, l);
-        if constexpr (V == 4)
-            lds_store_unit<1>(lds, q, 0, l);
-        else
-            store_state<V>(lds, q, l);
-    }
-    __syncthreads();
-    const int pos = threadIdx.x;
+    const int pos = threadIdx.x, lane = pos & 63;
     const int64_t i = t * kBlock + a.rowb[t * kBlock + pos];
-    if (i >= a.N) return;
-    const int lane = pos & 63;
-    const int64_t sl = t * (kBlock / kSellC) + (pos >> 6);
+    const int64_t sl = t * (kBlock / kSellC) + __builtin_amdgcn_readfirstlane(pos >> 6);
     const int64_t off = a.sb_off[sl];
     const int W = a.sb_w[sl];
+    struct Batch {
+        int32_t r[BT];
+        double2 w[BT];
+    };
+    auto load = [&](int e0, Batch& q) {
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+            const int64_t at = off + (int64_t)((e0 + b < W) ? e0 + b : e0) * kSellC + lane;
+            q.r[b] = a.lb[at];
+            q.w[b] = a.twb[at];
+        }
+    };
+    Batch q0, q1;
+    if (W > 0) load(0, q0);
+    VjpTail<V> tail;
+    if (AHEAD && i < a.N) load_tail<V>(a, i, tail);
+    struct Lam {
+        double l[V];
+        uint32_t f;
+    };
+    auto get = [&](int64_t r, Lam& x) {
+        load_state<V>(a.lam, r, x.l);
+        x.f = a.flag ? a.flag[r] : 0u;
+    };
+    for_halo<kHaloLoads, Lam>(nh, a.hb_ids + h0, get, [&](int q, Lam& x) {
+        mask_lam<V>(x.f, x.l);
+        if constexpr (V == 4)
+            lds_store_unit<1>(lds, q, 0, x.l);
+        else
+            store_state<V>(lds, q, x.l);
+    });
+    __syncthreads();
+    if (i >= a.N) return;
     double gx[V], gy[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) gx[v] = gy[v] = 0.0;
-#pragma unroll 1
-    for (int e0 = 0; e0 < W; e0 += BT) {
-        int32_t r[BT];
-        double2 w[BT];
-#pragma unroll
-        for (int b = 0; b < BT; ++b) {
-            const int e = (e0 + b < W) ? e0 + b : e0;
-            const int64_t q = off + (int64_t)e * kSellC + lane;
-            r[b] = a.lb[q];
-            w[b] = a.twb[q];
-        }
+    auto use = [&](int e0, const Batch& q) {
         double l[BT][V];
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             if constexpr (V == 4)
-                lds_load_unit<1>(lds, r[b], 0, l[b]);
+                lds_load_unit<1>(lds, q.r[b], 0, l[b]);
             else
-                load_state<V>(lds, r[b], l[b]);
+                load_state<V>(lds, q.r[b], l[b]);
         }
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             if (e0 + b >= W) continue;
 #pragma unroll
             for (int v = 0; v < V; ++v) {
-                gx[v] = fma(w[b].x, l[b][v], gx[v]);
-                gy[v] = fma(w[b].y, l[b][v], gy[v]);
+                gx[v] = fma(q.w[b].x, l[b][v], gx[v]);
+                gy[v] = fma(q.w[b].y, l[b][v], gy[v]);
             }
         }
+    };
+#pragma unroll 1
+    for (int e0 = 0; e0 < W; e0 += 2 * BT) {
+        if (e0 + BT < W) load(e0 + BT, q1);
+        __builtin_amdgcn_sched_barrier(0);
+        use(e0, q0);
+        if (e0 + 2 * BT < W) load(e0 + 2 * BT, q0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (e0 + BT < W) use(e0 + BT, q1);
     }
-    vjp_finish<V>(a, i, gx, gy);
+    if constexpr (!AHEAD) load_tail<V>(a, i, tail);
+    vjp_finish<V>(a, i, tail, gx, gy);
 }
 
 static VjpArgs vjp_args(mf_ctx* c)
@@ -256,10 +292,14 @@ static int launch_vjp(mf_ctx* c, const VjpArgs& a)
     if (c->tiles_b) {
         // halo records of nvar doubles (the tiles were sized for at least that)
         const size_t lds = (size_t)c->hb_max * c->nvar * sizeof(double);
-        if (c->nvar == 4)
-            hipLaunchKernelGGL((k_vjp_tl<4, 8>), dim3(grid), dim3(kBlock), lds, c->stream, a);
-        else
-            hipLaunchKernelGGL((k_vjp_tl<1, 8>), dim3(grid), dim3(kBlock), lds, c->stream, a);
+        // Four values: batches of 8 and the node's values held where the tiles
+        // do not fill the CUs (a step and its adjoint, K = 30: 50.4 against
+        // 52.0 us at 126 tiles, 65.2 / 66.8 at 256), batches of 4 beyond,
+        // where their wavefronts count (83.9 / 82.8 at 351, 123.8 / 111.1 at
+        // 514, 175.2 / 174.9 at 1024).  One value: no difference.
+        const bool small = c->n_tiles <= c->cu_count;
+        auto k = c->nvar == 1 ? k_vjp_tl<1, 8, false> : small ? k_vjp_tl<4, 8, true> : k_vjp_tl<4, 4, false>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), lds, c->stream, a);
     } else if (c->nvar == 4) {
         hipLaunchKernelGGL(k_vjp<4>, dim3(grid), dim3(kBlock), 0, c->stream, a);
     } else {
@@ -270,20 +310,43 @@ static int launch_vjp(mf_ctx* c, const VjpArgs& a)
 }
 
 // L = sum_i rho_i^2 over the (boundary-imposed) state and its gradient
-// dL/du = (2 rho, 0, ...).
-__global__ void k_loss(int64_t N, int V, const double* u, double* grad, double* loss)
+// dL/du = (2 rho, 0, ...).  1024 running sums, each over every 1024th node in
+// ascending order, then a tree over them.  One block of 1024 threads did both
+// and waited for one node at a time (95 us at 65,536 nodes of four values);
+// each wavefront of 64 sums is now a block of its own with kLossLoads nodes of
+// each sum in flight, and a second kernel adds them up
+// (10.6 and 2.8 us).
+constexpr int kLossSums = 1024, kLossLoads = 16;
+
+__global__ __launch_bounds__(64) void k_loss_sums(int64_t N, int V, const double* u, double* grad, double* sums)
 {
-    __shared__ double red[1024];
+    const int s = blockIdx.x * 64 + threadIdx.x;
     double acc = 0.0;
-    for (int64_t i = threadIdx.x; i < N; i += blockDim.x) {
-        const double r = u[i * V];
-        acc = fma(r, r, acc);
-        grad[i * V] = 2.0 * r;
-        for (int v = 1; v < V; ++v) grad[i * V + v] = 0.0;
+    for (int64_t i0 = s; i0 < N; i0 += (int64_t)kLossSums * kLossLoads) {
+        double r[kLossLoads];
+#pragma unroll
+        for (int q = 0; q < kLossLoads; ++q) {
+            const int64_t i = i0 + (int64_t)q * kLossSums;
+            r[q] = u[(i < N ? i : i0) * V];
+        }
+#pragma unroll
+        for (int q = 0; q < kLossLoads; ++q) {
+            const int64_t i = i0 + (int64_t)q * kLossSums;
+            if (i >= N) continue;
+            acc = fma(r[q], r[q], acc);
+            grad[i * V] = 2.0 * r[q];
+            for (int v = 1; v < V; ++v) grad[i * V + v] = 0.0;
+        }
     }
-    red[threadIdx.x] = acc;
+    sums[s] = acc;
+}
+
+__global__ __launch_bounds__(kLossSums) void k_loss(const double* sums, double* loss)
+{
+    __shared__ double red[kLossSums];
+    red[threadIdx.x] = sums[threadIdx.x];
     __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+    for (int w = kLossSums / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
@@ -366,12 +429,14 @@ int mf_ssprk33_vjp(mf_ctx* c, double t0, double dt, int n_steps, int checkpoint_
     const int64_t NV = c->N * c->nvar;
     // buffers: checkpoints, 3 tape states per step of a segment, Ubar, Sbar2, Sbar1, two work states
     const int64_t nbuf = nck + 3 * (int64_t)C + 6;
-    if (c->adj_len < nbuf * NV) {
+    // and the sums of the loss after them
+    const int64_t len = nbuf * NV + kLossSums + 1;
+    if (c->adj_len < len) {
         dfree(c->d_adj);
         c->d_adj = nullptr;
         c->adj_len = 0;
-        if ((rc = dalloc(c, &c->d_adj, (size_t)(nbuf * NV)))) return rc;
-        c->adj_len = nbuf * NV;
+        if ((rc = dalloc(c, &c->d_adj, (size_t)len))) return rc;
+        c->adj_len = len;
     }
     // checkpoint s at buf(s); the tape and work states after them
     auto buf = [&](int64_t q) { return c->d_adj + q * NV; };
@@ -438,8 +503,10 @@ int mf_ssprk33_vjp(mf_ctx* c, double t0, double dt, int n_steps, int checkpoint_
     // loss on the final state (W1) after its boundary pass (the last FSAL call)
     time.set(tn[n_steps]);
     if (!hand && (rc = bc_pass_state(c, W1, 0.0))) return rc;
-    double* d_loss = W0;
-    hipLaunchKernelGGL(k_loss, dim3(1), dim3(1024), 0, c->stream, c->N, c->nvar, W1, Ub, d_loss);
+    double *sums = buf(nbuf), *d_loss = sums + kLossSums;
+    hipLaunchKernelGGL(k_loss_sums, dim3(kLossSums / 64), dim3(64), 0, c->stream, c->N, c->nvar, W1, Ub, sums);
+    MF_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_loss, dim3(1), dim3(kLossSums), 0, c->stream, sums, d_loss);
     MF_HIP(c, hipGetLastError());
     double hl = 0.0;
     MF_HIP(c, hipMemcpyAsync(&hl, d_loss, sizeof(double), hipMemcpyDeviceToHost, c->stream));

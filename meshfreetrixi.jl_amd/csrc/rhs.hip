@@ -214,13 +214,62 @@ __device__ __forceinline__ void load_state32(const float* __restrict__ p, int64_
     }
 }
 
+// What the end of a kernel reads of its node: the boundary flag and, for a
+// stage, the node's input state, the previous state and the boundary entry.
+// The kernels of small grids (the stencil kernels with two batches in flight,
+// the transposed one with batches of 8) load it ahead of the row's entries,
+// so that it arrives while they are summed: after the sums it was one more
+// wait for memory.  On large grids the other wavefronts cover that wait, and
+// the registers held through the sums would cost wavefronts (V = 4, K = 30,
+// FP64 in batches of 3: 78 -> 106 VGPRs, four per SIMD instead of six).
+template <int V, bool AHEAD>
+struct NodeTail {
+    double u[V], up[V];
+    uint32_t flag;
+    int32_t oent;
+};
+
+// Loads the values if they are held (AHEAD); otherwise they are loaded where
+// they are used.  The flag is read only with a.flag set.
+template <int V, bool AHEAD>
+__device__ __forceinline__ void load_tail(const RhsArgs& a, int64_t i, NodeTail<V, AHEAD>& t)
+{
+    if constexpr (!AHEAD) return;
+    t.flag = a.flag ? a.flag[i] : 0u;
+    t.oent = -1;
+    if (a.st_kind == ST_NONE) return;
+    load_state<V>(a.u, i, t.u);
+    if (a.st_kind != ST_FSAL) load_state<V>(a.uprev, i, t.up);
+    if (a.obc.flag) t.oent = a.obc.entry[i];
+}
+
+template <int V, bool AHEAD>
+__device__ __forceinline__ uint32_t tail_flag(const RhsArgs& a, int64_t i, const NodeTail<V, AHEAD>& t)
+{
+    if constexpr (AHEAD)
+        return t.flag;
+    else
+        return a.flag[i];
+}
+
+template <int V, bool AHEAD>
+__device__ __forceinline__ void tail_state(const double* held, const double* __restrict__ p, int64_t i, double* s)
+{
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) s[v] = held[v];
+    } else {
+        load_state<V>(p, i, s);
+    }
+}
+
 // Second boundary pass on du (rbfsolver.jl:422-425): Dirichlet nodes get
 // du = 0, slip nodes du momentum = 0.
-template <int V>
-__device__ __forceinline__ void mask_du(const RhsArgs& a, int64_t i, double* du)
+template <int V, bool AHEAD>
+__device__ __forceinline__ void mask_du(const RhsArgs& a, int64_t i, const NodeTail<V, AHEAD>& t, double* du)
 {
     if (!a.flag) return;
-    const uint8_t f = a.flag[i];
+    const uint32_t f = tail_flag(a, i, t);
     if (f & 1u) {
 #pragma unroll
         for (int v = 0; v < V; ++v) du[v] = 0.0;
@@ -239,20 +288,21 @@ __device__ __forceinline__ void mask_du(const RhsArgs& a, int64_t i, double* du)
 //   THREE: out = (uprev + 2 u + 2 dt k) / 3
 // u is this node's (boundary-imposed) input state; slip nodes see the
 // second boundary pass's projection first, as the reference's u does.
-template <int V>
-__device__ __forceinline__ void stage_value(const RhsArgs& a, int64_t i, const double* du, double* o)
+template <int V, bool AHEAD>
+__device__ __forceinline__ void stage_value(const RhsArgs& a, int64_t i, const NodeTail<V, AHEAD>& t,
+                                            const double* du, double* o)
 {
     double ui[V];
-    load_state<V>(a.u, i, ui);
+    tail_state<V, AHEAD>(t.u, a.u, i, ui);
     if constexpr (V == 4) {
-        if (a.flag && (a.flag[i] & 2u)) slip_project(a.bnormal + 2 * a.entry[i], ui);
+        if (a.flag && (tail_flag(a, i, t) & 2u)) slip_project(a.bnormal + 2 * a.entry[i], ui);
     }
     if (a.st_kind == ST_FSAL) {
 #pragma unroll
         for (int v = 0; v < V; ++v) o[v] = fma(a.dt, du[v], ui[v]);
     } else {
         double up[V];
-        load_state<V>(a.uprev, i, up);
+        tail_state<V, AHEAD>(t.up, a.uprev, i, up);
         if (a.st_kind == ST_TWO) {
 #pragma unroll
             for (int v = 0; v < V; ++v) o[v] = fma(3.0, up[v], fma(a.dt, du[v], ui[v])) / 4.0;
@@ -266,16 +316,21 @@ __device__ __forceinline__ void stage_value(const RhsArgs& a, int64_t i, const d
 
 // The output of node i: du, or the next stage with, in stepping, the first
 // boundary pass of the rhs! that reads it; o returns the stored stage.
-template <int V>
-__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* du, double* o)
+template <int V, bool AHEAD>
+__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const NodeTail<V, AHEAD>& t, const double* du,
+                                     double* o)
 {
     if (a.st_kind == ST_NONE) {
         store_state<V>(a.du, i, du);
         return;
     }
-    stage_value<V>(a, i, du, o);
+    stage_value(a, i, t, du, o);
     if (a.obc.flag) {
-        const int32_t e = a.obc.entry[i];
+        int32_t e;
+        if constexpr (AHEAD)
+            e = t.oent;
+        else
+            e = a.obc.entry[i];
         if (e >= 0) {
             if (a.sraw) store_state<V>(a.sraw, e, o);
             bc_node<V>(a.obc, e, (int32_t)i, o);
@@ -284,11 +339,11 @@ __device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* 
     store_state<V>(a.out, i, o);
 }
 
-template <int V>
-__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const double* du)
+template <int V, bool AHEAD>
+__device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const NodeTail<V, AHEAD>& t, const double* du)
 {
     double o[V];
-    emit<V>(a, i, du, o);
+    emit(a, i, t, du, o);
 }
 
 // Residual/upwind viscosity at node i (hyperviscosity.jl:246-349): eps_uw
@@ -465,10 +520,13 @@ __device__ __forceinline__ void stage_halo_a(const RhsArgs& a, int64_t t, double
     if constexpr (TL) {
         const int64_t h0 = a.ha_off[t];
         const int nh = (int)(a.ha_off[t + 1] - h0);
-        for (int q = threadIdx.x; q < nh; q += kBlock) {
-            double s[V], r[rec_len<V>()];
-            load_state<V>(a.u, a.ha_ids[h0 + q], s);
-            make_record<V>(a.eq, s, r);
+        struct State {
+            double s[V];
+        };
+        auto get = [&](int32_t j, State& s) { load_state<V>(a.u, j, s.s); };
+        for_halo<kHaloLoads, State>(nh, a.ha_ids + h0, get, [&](int q, const State& s) {
+            double r[rec_len<V>()];
+            make_record<V>(a.eq, s.s, r);
             if constexpr (V == 4) {
                 double2* p = reinterpret_cast<double2*>(lds) + 3 * q;
                 p[0] = make_double2(r[0], r[1]);
@@ -477,7 +535,7 @@ __device__ __forceinline__ void stage_halo_a(const RhsArgs& a, int64_t t, double
             } else {
                 store_state<V>(lds, q, r);
             }
-        }
+        });
         if (rvres) {
             wave_lexmax4(pm);
             store_wave4(pm, wmax);
@@ -626,6 +684,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
             }
         }
     };
+    NodeTail<V, PF> tail;
+    if constexpr (!RV && !TOM) load_tail(a, i, tail);
     for_batches<BT, PF>(K, q0, load, use);
     double du[V];
 #pragma unroll
@@ -664,8 +724,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
         store_state<V>(a.du, i, du);
         return;
     }
-    mask_du<V>(a, i, du);
-    emit<V>(a, i, du);
+    mask_du(a, i, tail, du);
+    emit(a, i, tail, du);
 }
 
 // --------------------------------------- FP64 in the reference's order
@@ -778,6 +838,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
     double du[V], gx[V], gy[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) du[v] = gx[v] = gy[v] = 0.0;
+    NodeTail<V, PF> tail;
+    if constexpr (!RV && !TOM) load_tail(a, i, tail);
     ref_pass<V, NS, RV, BT, PF, 0, TL>(a, blk, i, K, du, gx, lds, a.wx_s, q0, a.wy_s);
     double ui[V], ad[V];  // the node's state and approx_du, in flight through the y pass
     if constexpr (RV) {
@@ -817,8 +879,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
         store_state<V>(a.du, i, du);
         return;
     }
-    mask_du<V>(a, i, du);
-    emit<V>(a, i, du);
+    mask_du(a, i, tail, du);
+    emit(a, i, tail, du);
 }
 
 // ------------------------------------------------- split-FP32 kernel
@@ -921,6 +983,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
             }
         }
     };
+    NodeTail<V, PF> tail;
+    if constexpr (!RV && !TOM) load_tail(a, i, tail);
     for_batches<BT, PF>(K, q0, load, use);
     double du[V];
 #pragma unroll
@@ -965,8 +1029,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
         store_state32<V>(a.du32, i, du);
         return;
     }
-    mask_du<V>(a, i, du);
-    emit<V>(a, i, du);
+    mask_du(a, i, tail, du);
+    emit(a, i, tail, du);
 }
 
 // ------------------------------------------ phase B: transposed gather
@@ -1041,34 +1105,43 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
         i = t * kBlock + a.rowb[t * kBlock + threadIdx.x];
         live = i < a.N;
         if (W > 0) load(0, q0);
-        for (int q = threadIdx.x; q < nh; q += kBlock) {
-            const int64_t j = a.hb_ids[h0 + q];
-            if constexpr (TM == 1) {  // FP32 records
-                float* ldsf = reinterpret_cast<float*>(lds);
-                double g[V];
+        if constexpr (TM == 1) {  // FP32 records
+            float* ldsf = reinterpret_cast<float*>(lds);
+            struct Rec {
+                double g0[V], g1[V], l[V];
+            };
+            auto get = [&](int64_t j, Rec& x) {
                 if constexpr (HG) {
-                    load_state32<V>(a.G32, 2 * j, g);
-                    lds_store_unit32<RU>(ldsf, q, 0, g);
-                    load_state32<V>(a.G32, 2 * j + 1, g);
-                    lds_store_unit32<RU>(ldsf, q, 1, g);
+                    load_state32<V>(a.G32, 2 * j, x.g0);
+                    load_state32<V>(a.G32, 2 * j + 1, x.g1);
                 }
-                if constexpr (HL) {
-                    load_state32<V>(a.L32, j, g);
-                    lds_store_unit32<RU>(ldsf, q, LU, g);
-                }
-            } else {
-                double g[V];
+                if constexpr (HL) load_state32<V>(a.L32, j, x.l);
+            };
+            for_halo<kHaloLoads, Rec>(nh, a.hb_ids + h0, get, [&](int q, const Rec& x) {
                 if constexpr (HG) {
-                    load_state<V>(a.G, 2 * j, g);
-                    lds_store_unit<RU>(lds, q, 0, g);
-                    load_state<V>(a.G, 2 * j + 1, g);
-                    lds_store_unit<RU>(lds, q, 1, g);
+                    lds_store_unit32<RU>(ldsf, q, 0, x.g0);
+                    lds_store_unit32<RU>(ldsf, q, 1, x.g1);
                 }
-                if constexpr (HL) {
-                    load_state<V>(a.L, j, g);
-                    lds_store_unit<RU>(lds, q, LU, g);
+                if constexpr (HL) lds_store_unit32<RU>(ldsf, q, LU, x.l);
+            });
+        } else {
+            struct Rec {
+                double g0[V], g1[V], l[V];
+            };
+            auto get = [&](int64_t j, Rec& x) {
+                if constexpr (HG) {
+                    load_state<V>(a.G, 2 * j, x.g0);
+                    load_state<V>(a.G, 2 * j + 1, x.g1);
                 }
-            }
+                if constexpr (HL) load_state<V>(a.L, j, x.l);
+            };
+            for_halo<kHaloLoads, Rec>(nh, a.hb_ids + h0, get, [&](int q, const Rec& x) {
+                if constexpr (HG) {
+                    lds_store_unit<RU>(lds, q, 0, x.g0);
+                    lds_store_unit<RU>(lds, q, 1, x.g1);
+                }
+                if constexpr (HL) lds_store_unit<RU>(lds, q, LU, x.l);
+            });
         }
         __syncthreads();
         if (!live && !a.stage_psum) return;
@@ -1085,6 +1158,17 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             if (W > 0) load(0, q0);  // a slice of nodes that no stencil names has no entries
         }
     }
+    constexpr bool kAhead = TL && BT > 4;  // see NodeTail
+    NodeTail<V, kAhead> tail;
+    double du[V];  // phase A's part
+    auto load_node = [&] {
+        load_tail(a, i, tail);
+        if constexpr (TM == 1)
+            load_state32<V>(a.du32, i, du);
+        else
+            load_state<V>(a.du, i, du);
+    };
+    if (kAhead && live) load_node();
     double tx[V], ty[V], th[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) tx[v] = ty[v] = th[v] = 0.0;
@@ -1161,11 +1245,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
     }
     double o[4] = {0.0, 0.0, 0.0, 0.0};  // the stored output (staged stages)
     if (live) {
-        double du[V];
-        if constexpr (TM == 1)
-            load_state32<V>(a.du32, i, du);
-        else
-            load_state<V>(a.du, i, du);
+        if constexpr (!kAhead) load_node();
         if constexpr (TM == 2) {
             // the phase-B sources in keyword order
             for (int sq = a.seq_b; sq != 0; sq >>= 2) {
@@ -1199,8 +1279,8 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
                 for (int v = 0; v < V; ++v) du[v] = fma(-a.tom_gamma, th[v], du[v]);
             }
         }
-        mask_du<V>(a, i, du);
-        emit<V>(a, i, du, o);
+        mask_du(a, i, tail, du);
+        emit(a, i, tail, du, o);
     }
     if constexpr (V == 4) {
         if (a.stage_psum) {  // the same for the whole block
@@ -1789,14 +1869,13 @@ __device__ __forceinline__ double2 igr_grad_tl(const IgrArgs& a, int64_t blk, co
     return make_double2(sx, sy);
 }
 
-// put(q, j) for every halo entry q of tile t (node j); ends with a block
-// barrier.
-template <class Put>
-__device__ __forceinline__ void igr_stage(const IgrArgs& a, int64_t t, Put put)
+// The halo of tile t by for_halo; ends with a block barrier.
+template <class T, class Get, class Put>
+__device__ __forceinline__ void igr_stage(const IgrArgs& a, int64_t t, Get get, Put put)
 {
     const int64_t h0 = a.ha_off[t];
     const int nh = (int)(a.ha_off[t + 1] - h0);
-    for (int q = threadIdx.x; q < nh; q += kBlock) put(q, a.ha_ids[h0 + q]);
+    for_halo<kHaloLoads, T>(nh, a.ha_ids + h0, get, put);
     __syncthreads();
 }
 
@@ -1816,13 +1895,16 @@ __global__ __launch_bounds__(kBlock) void k_igr_init(const IgrArgs a)
     IgrBatch q0;
     if constexpr (TL) {
         igr_load(a, lb, 0, q0);
-        igr_stage(a, lb, [&](int q, int32_t j) {
+        struct State {
             double u[4];
-            load_state<4>(a.u, j, u);
-            lds[3 * q] = u[0];
-            lds[3 * q + 1] = u[1] / u[0];
-            lds[3 * q + 2] = u[2] / u[0];
-        });
+        };
+        igr_stage<State>(
+            a, lb, [&](int32_t j, State& s) { load_state<4>(a.u, j, s.u); },
+            [&](int q, const State& s) {
+                lds[3 * q] = s.u[0];
+                lds[3 * q + 1] = s.u[1] / s.u[0];
+                lds[3 * q + 2] = s.u[2] / s.u[0];
+            });
     }
     double rr = 0.0;
     if (i < a.N) {
@@ -2003,9 +2085,9 @@ __global__ __launch_bounds__(kBlock) void k_igr_c_tl(const IgrArgs a)
         ri = a.rinv[i];
         pi = a.p[i];
     }
-    igr_stage(a, lb, [&](int q, int32_t j) {
-        reinterpret_cast<double2*>(lds)[q] = make_double2(a.t1[j], a.t2[j]);
-    });
+    igr_stage<double2>(
+        a, lb, [&](int32_t j, double2& v) { v = make_double2(a.t1[j], a.t2[j]); },
+        [&](int q, const double2& v) { reinterpret_cast<double2*>(lds)[q] = v; });
     if (done) return;
     double pc = 0.0;
     if (i < a.N) {
@@ -2060,21 +2142,26 @@ __global__ __launch_bounds__(kBlock) void k_igr_apply(const IgrArgs g, const Rhs
     if (lb >= g.nblk) return;  // whole block
     const int64_t i = lb * kBlock + threadIdx.x;
     double2 s = make_double2(0.0, 0.0);
+    NodeTail<4, TL> tail;
+    double du[4];
+    if (i < g.N) {
+        load_tail(a, i, tail);
+        load_state<4>(a.du, i, du);
+    }
     if constexpr (TL) {
         IgrBatch q0;
         igr_load(g, lb, 0, q0);
-        igr_stage(g, lb, [&](int q, int32_t j) { lds[q] = g.x[j]; });
+        igr_stage<double>(
+            g, lb, [&](int32_t j, double& v) { v = g.x[j]; }, [&](int q, const double& v) { lds[q] = v; });
         if (i < g.N) s = igr_grad_tl<false>(g, lb, lds, q0);
     } else {
         if (i < g.N) s = igr_grad<5>(g, i, g.x);
     }
     if (i >= g.N) return;
-    double du[4];
-    load_state<4>(a.du, i, du);
     du[1] -= s.x;
     du[2] -= s.y;
-    mask_du<4>(a, i, du);
-    emit<4>(a, i, du);
+    mask_du(a, i, tail, du);
+    emit(a, i, tail, du);
 }
 
 static IgrArgs make_igr(mf_ctx* c, const double* u)
