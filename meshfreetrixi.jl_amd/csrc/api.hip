@@ -179,8 +179,9 @@ static void free_state(mf_ctx* c)
     dfree(c->d_partials);
     dfree(c->d_stage_psum);
     dfree(c->d_lim);
+    dfree(c->d_lim2);
     dfree(c->d_adj);
-    c->d_S = c->d_T = c->d_G = c->d_eps = c->d_approx = c->d_hist = c->d_partials = c->d_lim = nullptr;
+    c->d_S = c->d_T = c->d_G = c->d_eps = c->d_approx = c->d_hist = c->d_partials = c->d_lim = c->d_lim2 = nullptr;
     c->d_stage_psum = nullptr;
     c->d_adj = nullptr;
     c->adj_len = 0;
@@ -255,7 +256,14 @@ int ensure_state(mf_ctx* c)
             return rc;
     }
     // limiter scratch: nvar N blended values, then N flag bytes
-    if (!c->d_lim && (rc = dalloc(c, &c->d_lim, nv + (size_t)(c->N + 7) / 8))) return rc;
+    const size_t lim_len = nv + (size_t)(c->N + 7) / 8;
+    if (!c->d_lim && (rc = dalloc(c, &c->d_lim, lim_len))) return rc;
+    if (c->lim_n > 1 && !c->d_lim2 && dalloc(c, &c->d_lim2, lim_len)) {
+        // without it each pass copies its rows back
+        c->d_lim2 = nullptr;
+        c->err.clear();
+        (void)hipGetLastError();
+    }
     return MF_OK;
 }
 
@@ -1304,7 +1312,7 @@ int mf_limiter_zhang_shu(mf_ctx* c, double threshold, int variable)
     if (variable != MF_VAR_DENSITY && variable != MF_VAR_PRESSURE) return fail(c, MF_ERR_ARGUMENT, "limiter: bad variable");
     if (variable == MF_VAR_PRESSURE && c->nvar != 4) return fail(c, MF_ERR_UNSUPPORTED, "limiter: pressure needs Euler");
     if ((rc = ensure_state(c))) return rc;
-    if ((rc = run_limiter(c, c->d_buf[MF_BUF_U], threshold, variable))) return rc;
+    if ((rc = run_limiter(c, c->d_buf[MF_BUF_U], 1, &threshold, &variable))) return rc;
     MF_HIP(c, hipStreamSynchronize(c->stream));
     return MF_OK;
 }
@@ -1350,11 +1358,7 @@ static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history
     int rc;
     auto limit = [&](double* u) -> int {
         if (!limiter) return MF_OK;
-        for (int q = 0; q < c->lim_n; ++q) {
-            int r2 = run_limiter(c, u, c->lim_thr[q], c->lim_var[q]);
-            if (r2) return r2;
-        }
-        return MF_OK;
+        return run_limiter(c, u, c->lim_n, c->lim_thr, c->lim_var);
     };
     double* U = c->d_buf[MF_BUF_U];
     if ((rc = limit(c->d_S))) return rc;

@@ -178,6 +178,7 @@ struct mf_ctx {
     double lim_thr[2] = {0, 0};
     int lim_var[2] = {0, 0};
     double* d_lim = nullptr;  // limiter scratch: nvar N values, then N flag bytes
+    double* d_lim2 = nullptr;  // the same for the second of two passes (null: no memory for it)
 
     // graph of one SSPRK33 step
     // graphs of one step and of kGraphSteps consecutive steps (fewer launches)
@@ -395,7 +396,7 @@ int run_set_time(mf_ctx* c, double t, int success_iter);
 int run_history(mf_ctx* c, const double* d_u, int init, double advance_dt = 0.0);
 // the boundary entries' raw values (d_sraw) back into d_u
 int run_restore_raw(mf_ctx* c, double* d_u);
-int run_limiter(mf_ctx* c, double* d_u, double thr, int var);
+int run_limiter(mf_ctx* c, double* d_u, int n, const double* thr, const int* var);
 // the first boundary pass (at the step's time + dt_off) and its transpose
 int bc_pass_state(mf_ctx* c, double* d_u, double dt_off);
 int bc_pass_homog(mf_ctx* c, double* d_u);

@@ -1589,6 +1589,53 @@ __device__ __forceinline__ double limiter_variable(int var, double gamma, const 
     return (gamma - 1.0) * (s[3] - 0.5 * (s[1] * s[1] + s[2] * s[2]) / s[0]);
 }
 
+// One limiter pass.  With ploc the state is that after an earlier pass whose
+// blended rows are not yet copied back: row j is ploc's where pflag is set, u's
+// otherwise, so two passes in a row need one copy after both of them and not
+// one after each (2.0 us of launch each at 17,161 nodes).
+struct LimArgs {
+    int64_t N;
+    int K;
+    const int32_t* __restrict__ idx;
+    const double* __restrict__ u;
+    double* __restrict__ loc;
+    uint8_t* __restrict__ flag;
+    const double* __restrict__ ploc;
+    const uint8_t* __restrict__ pflag;
+    double thr;
+    int var;
+    double gamma;
+    // LDS tiles of the stencil kernel
+    const uint16_t* __restrict__ la;
+    int64_t n_tiles;
+    const int64_t* __restrict__ ha_off;
+    const int32_t* __restrict__ ha_ids;
+};
+
+template <int V>
+__device__ __forceinline__ void limiter_state(const LimArgs& a, int64_t j, double* s)
+{
+    const uint32_t f = a.ploc ? a.pflag[j] : 0u;
+    load_state<V>(a.u, j, s);
+    if (f) load_state<V>(a.ploc, j, s);
+}
+
+// The limited variable of node j: density alone needs only the first
+// component.
+template <int V>
+__device__ __forceinline__ double limiter_value(const LimArgs& a, int64_t j)
+{
+    if (a.var == MF_VAR_DENSITY || V == 1) {
+        const uint32_t f = a.ploc ? a.pflag[j] : 0u;
+        double v = a.u[j * V];
+        if (f) v = a.ploc[j * V];
+        return v;
+    }
+    double s[V];
+    limiter_state<V>(a, j, s);
+    return limiter_variable<V>(a.var, a.gamma, s);
+}
+
 // Stencil entries per load batch of the minimum: the batch's index loads,
 // then its neighbour loads, are all in flight together.
 constexpr int kLimBatch = 10;
@@ -1596,28 +1643,26 @@ constexpr int kLimBatch = 10;
 // Node i with stencil minimum vmin below the threshold: the theta-blend with
 // the stencil mean (in stencil order) into loc, and the row's flag byte.
 template <int V>
-__device__ __forceinline__ void limiter_finish(int64_t N, int K, const int32_t* idx, const double* u,
-                                               double* loc, uint8_t* flag, double thr, int var, double gamma,
-                                               int64_t i, double vmin)
+__device__ __forceinline__ void limiter_finish(const LimArgs& a, int64_t i, double vmin)
 {
     uint8_t f = 0;
-    if (vmin < thr) {
+    if (vmin < a.thr) {
         double o[V];
         double um[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) um[v] = 0.0;
-        for (int s = 0; s < K; ++s) {
+        for (int s = 0; s < a.K; ++s) {
             double uj[V];
-            load_state<V>(u, idx[(int64_t)s * N + i], uj);
+            limiter_state<V>(a, a.idx[(int64_t)s * a.N + i], uj);
 #pragma unroll
             for (int v = 0; v < V; ++v) um[v] = um[v] + uj[v];
         }
 #pragma unroll
-        for (int v = 0; v < V; ++v) um[v] = um[v] / (double)K;
-        const double vmean = limiter_variable<V>(var, gamma, um);
-        const double theta = (vmean - thr) / (vmean - vmin);
+        for (int v = 0; v < V; ++v) um[v] = um[v] / (double)a.K;
+        const double vmean = limiter_variable<V>(a.var, a.gamma, um);
+        const double theta = (vmean - a.thr) / (vmean - vmin);
         double ui[V];
-        load_state<V>(u, i, ui);
+        limiter_state<V>(a, i, ui);
 #pragma unroll
         for (int v = 0; v < V; ++v) o[v] = fma(theta, ui[v], (1.0 - theta) * um[v]);
         // only non-zero rows are copied back (a row of zeros stays unwritten)
@@ -1625,99 +1670,97 @@ __device__ __forceinline__ void limiter_finish(int64_t N, int K, const int32_t* 
 #pragma unroll
         for (int v = 0; v < V; ++v) nz |= (o[v] != 0.0);
         if (nz) {
-            store_state<V>(loc, i, o);
+            store_state<V>(a.loc, i, o);
             f = 1;
         }
     }
-    flag[i] = f;
+    a.flag[i] = f;
 }
 
 template <int V>
-__global__ __launch_bounds__(kBlock) void k_limiter_blend(int64_t N, int K, const int32_t* idx,
-                                                          const double* u, double* loc, uint8_t* flag,
-                                                          double thr, int var, double gamma)
+__global__ __launch_bounds__(kBlock) void k_limiter_blend(const LimArgs a)
 {
     const int64_t i = remapped_node();
-    if (i >= N) return;
-    // the limited variable of every stencil node: density alone needs only
-    // the first component of each neighbour
-    const bool dens = var == MF_VAR_DENSITY || V == 1;
+    if (i >= a.N) return;
     double vmin = INFINITY;
 #pragma unroll 1
-    for (int s0 = 0; s0 < K; s0 += kLimBatch) {
+    for (int s0 = 0; s0 < a.K; s0 += kLimBatch) {
         int32_t j[kLimBatch];
 #pragma unroll
-        for (int b = 0; b < kLimBatch; ++b) j[b] = (s0 + b < K) ? idx[(int64_t)(s0 + b) * N + i] : (int32_t)i;
+        for (int b = 0; b < kLimBatch; ++b) j[b] = (s0 + b < a.K) ? a.idx[(int64_t)(s0 + b) * a.N + i] : (int32_t)i;
         double val[kLimBatch];
-        if (dens) {
 #pragma unroll
-            for (int b = 0; b < kLimBatch; ++b) val[b] = u[(int64_t)j[b] * V];
-        } else {
-#pragma unroll
-            for (int b = 0; b < kLimBatch; ++b) {
-                double uj[V];
-                load_state<V>(u, j[b], uj);
-                val[b] = limiter_variable<V>(var, gamma, uj);
-            }
-        }
+        for (int b = 0; b < kLimBatch; ++b) val[b] = limiter_value<V>(a, j[b]);
 #pragma unroll
         for (int b = 0; b < kLimBatch; ++b)
-            if (s0 + b < K) vmin = (val[b] < vmin) ? val[b] : vmin;
+            if (s0 + b < a.K) vmin = (val[b] < vmin) ? val[b] : vmin;
     }
-    limiter_finish<V>(N, K, idx, u, loc, flag, thr, var, gamma, i, vmin);
+    limiter_finish<V>(a, i, vmin);
 }
 
 // The same with the tile's stencil halo in LDS (the tiles of the stencil
 // kernel): the limited variable of every halo node is evaluated once into
 // LDS and the minimum reads it through the 16-bit halo positions la.  Same
-// values, same order, same bits.
+// values, same order, same bits.  Bound by its chain of waits for memory on
+// small grids: the first two batches of positions (every one up to K = 32) are
+// in flight while the halo is staged (17,161 nodes, K = 20: 5.7 -> 5.1 us).
 template <int V>
-__global__ __launch_bounds__(kBlock) void k_limiter_blend_tl(int64_t N, int K, const int32_t* idx,
-                                                             const uint16_t* la, int64_t n_tiles,
-                                                             const int64_t* ha_off, const int32_t* ha_ids,
-                                                             const double* u, double* loc, uint8_t* flag,
-                                                             double thr, int var, double gamma)
+__global__ __launch_bounds__(kBlock) void k_limiter_blend_tl(const LimArgs a)
 {
     extern __shared__ double lvar[];
     const int64_t t = remapped_block();
-    if (t >= n_tiles) return;  // whole block
-    const bool dens = var == MF_VAR_DENSITY || V == 1;
-    const int64_t h0 = ha_off[t];
-    const int nh = (int)(ha_off[t + 1] - h0);
-    for (int q = threadIdx.x; q < nh; q += kBlock) {
-        const int32_t j = ha_ids[h0 + q];
-        if (dens) {
-            lvar[q] = u[(int64_t)j * V];
-        } else {
-            double uj[V];
-            load_state<V>(u, j, uj);
-            lvar[q] = limiter_variable<V>(var, gamma, uj);
-        }
-    }
+    if (t >= a.n_tiles) return;  // whole block
+    constexpr int BT = 16;
+    struct Batch {
+        int32_t j[BT];
+    };
+    Batch q0, q1;
+    auto load = [&](int s0, Batch& q) {
+#pragma unroll
+        for (int b = 0; b < BT; ++b)
+            q.j[b] = s0 + b < a.K ? (int32_t)entry_of<true>(a.la, t, a.K, s0 + b, 0, 0) : 0;
+    };
+    load(0, q0);
+    load(BT, q1);
+    const int64_t h0 = a.ha_off[t];
+    const int nh = (int)(a.ha_off[t + 1] - h0);
+    for_halo<kHaloLoads, double>(
+        nh, a.ha_ids + h0, [&](int32_t j, double& v) { v = limiter_value<V>(a, j); },
+        [&](int q, const double& v) { lvar[q] = v; });
     __syncthreads();
     const int64_t i = t * kBlock + threadIdx.x;
-    if (i >= N) return;
+    if (i >= a.N) return;
     double vmin = INFINITY;
+    auto use = [&](int s0, const Batch& q) {
+        double val[BT];
+#pragma unroll
+        for (int b = 0; b < BT; ++b) val[b] = lvar[q.j[b]];
+#pragma unroll
+        for (int b = 0; b < BT; ++b)
+            if (s0 + b < a.K) vmin = (val[b] < vmin) ? val[b] : vmin;
+    };
 #pragma unroll 1
-    for (int s0 = 0; s0 < K; s0 += kLimBatch) {
-        double val[kLimBatch];
-#pragma unroll
-        for (int b = 0; b < kLimBatch; ++b) val[b] = lvar[(s0 + b < K) ? la[tm_pos(s0 + b, i, K)] : 0];
-#pragma unroll
-        for (int b = 0; b < kLimBatch; ++b)
-            if (s0 + b < K) vmin = (val[b] < vmin) ? val[b] : vmin;
+    for (int s0 = 0; s0 < a.K; s0 += 2 * BT) {
+        use(s0, q0);
+        if (s0 + BT < a.K) use(s0 + BT, q1);
+        if (s0 + 2 * BT < a.K) {
+            load(s0 + 2 * BT, q0);
+            load(s0 + 3 * BT, q1);
+        }
     }
-    limiter_finish<V>(N, K, idx, u, loc, flag, thr, var, gamma, i, vmin);
+    limiter_finish<V>(a, i, vmin);
 }
 
+// The blended rows into u: the last pass's, else those of the pass before it.
 template <int V>
-__global__ __launch_bounds__(kBlock) void k_limiter_commit(int64_t N, const double* loc, const uint8_t* flag,
-                                                           double* u)
+__global__ __launch_bounds__(kBlock) void k_limiter_commit(const LimArgs a, double* u)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N || !flag[i]) return;
+    if (i >= a.N) return;
+    const uint32_t f = a.flag[i], pf = a.ploc ? a.pflag[i] : 0u;
+    if (!f && !pf) return;
     double o[V];
-    load_state<V>(loc, i, o);
+    load_state<V>(f ? a.loc : a.ploc, i, o);
     store_state<V>(u, i, o);
 }
 
@@ -2711,39 +2754,42 @@ int run_history(mf_ctx* c, const double* d_u, int init, double advance_dt)
     return MF_OK;
 }
 
-int run_limiter(mf_ctx* c, double* d_u, double thr, int var)
+// The n limiter passes (at most two) over d_u in order.
+int run_limiter(mf_ctx* c, double* d_u, int n, const double* thr, const int* var)
 {
     const int64_t nblk = (c->N + kBlock - 1) / kBlock;
-    const unsigned grid = xcd_grid(nblk);
-    const double gam = c->p0;
-    // blended rows, then one flag byte per node (the buffer's tail)
-    uint8_t* flag = reinterpret_cast<uint8_t*>(c->d_lim + (int64_t)c->nvar * c->N);
-    if (c->tiles_a && c->d_la) {
-        // the stencil kernel's tiles: one LDS double per halo entry
-        const size_t lds = sizeof(double) * (size_t)c->ha_max;
-        const unsigned tg = xcd_grid(c->n_tiles);
-        if (c->nvar == 4)
-            hipLaunchKernelGGL(k_limiter_blend_tl<4>, dim3(tg), dim3(kBlock), lds, c->stream, c->N, c->k, c->d_idx,
-                               c->d_la, c->n_tiles, c->d_ha_off, c->d_ha_ids, d_u, c->d_lim, flag, thr, var, gam);
+    const bool tl = c->tiles_a && c->d_la;
+    const dim3 grid(xcd_grid(tl ? c->n_tiles : nblk)), block(kBlock);
+    // the stencil kernel's tiles: one LDS double per halo entry
+    const size_t lds = tl ? sizeof(double) * (size_t)c->ha_max : 0;
+    const int64_t NV = (int64_t)c->nvar * c->N;
+    LimArgs a{};
+    a.N = c->N;
+    a.K = c->k;
+    a.idx = c->d_idx;
+    a.u = d_u;
+    a.gamma = c->p0;
+    a.la = c->d_la;
+    a.n_tiles = c->n_tiles;
+    a.ha_off = c->d_ha_off;
+    a.ha_ids = c->d_ha_ids;
+    for (int q = 0; q < n; ++q) {
+        // blended rows, then one flag byte per node (the buffer's tail); with
+        // a second buffer the second pass reads the first one's rows from it
+        const bool second = q == 1 && c->d_lim2;
+        a.ploc = second ? a.loc : nullptr;
+        a.pflag = second ? a.flag : nullptr;
+        a.loc = second ? c->d_lim2 : c->d_lim;
+        a.flag = reinterpret_cast<uint8_t*>(a.loc + NV);
+        a.thr = thr[q];
+        a.var = var[q];
+        if (tl)
+            hipLaunchKernelGGL(c->nvar == 4 ? k_limiter_blend_tl<4> : k_limiter_blend_tl<1>, grid, block, lds, c->stream, a);
         else
-            hipLaunchKernelGGL(k_limiter_blend_tl<1>, dim3(tg), dim3(kBlock), lds, c->stream, c->N, c->k, c->d_idx,
-                               c->d_la, c->n_tiles, c->d_ha_off, c->d_ha_ids, d_u, c->d_lim, flag, thr, var, gam);
-        if (c->nvar == 4)
-            hipLaunchKernelGGL(k_limiter_commit<4>, dim3((unsigned)nblk), dim3(kBlock), 0, c->stream, c->N,
-                               c->d_lim, flag, d_u);
-        else
-            hipLaunchKernelGGL(k_limiter_commit<1>, dim3((unsigned)nblk), dim3(kBlock), 0, c->stream, c->N,
-                               c->d_lim, flag, d_u);
-    } else if (c->nvar == 4) {
-        hipLaunchKernelGGL(k_limiter_blend<4>, dim3(grid), dim3(kBlock), 0, c->stream, c->N, c->k,
-                           c->d_idx, d_u, c->d_lim, flag, thr, var, gam);
-        hipLaunchKernelGGL(k_limiter_commit<4>, dim3((unsigned)nblk), dim3(kBlock), 0, c->stream,
-                           c->N, c->d_lim, flag, d_u);
-    } else {
-        hipLaunchKernelGGL(k_limiter_blend<1>, dim3(grid), dim3(kBlock), 0, c->stream, c->N, c->k,
-                           c->d_idx, d_u, c->d_lim, flag, thr, var, gam);
-        hipLaunchKernelGGL(k_limiter_commit<1>, dim3((unsigned)nblk), dim3(kBlock), 0, c->stream,
-                           c->N, c->d_lim, flag, d_u);
+            hipLaunchKernelGGL(c->nvar == 4 ? k_limiter_blend<4> : k_limiter_blend<1>, grid, block, 0, c->stream, a);
+        if (q + 1 < n && c->d_lim2) continue;  // copied back with the next pass's
+        hipLaunchKernelGGL(c->nvar == 4 ? k_limiter_commit<4> : k_limiter_commit<1>, dim3((unsigned)nblk), block, 0,
+                           c->stream, a, d_u);
     }
     MF_HIP(c, hipGetLastError());
     return MF_OK;
