@@ -2544,20 +2544,29 @@ static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool r
 }
 
 // gt bit 0: G of the viscosity source, bit 1: L of the Tominec source (its
-// variants exist for the default batch only).
+// variants take no tuning).
 template <int TM, bool TL>
 static void launch_transpose_tl(mf_ctx* c, const RhsArgs& a, unsigned grid, size_t lds, int gt)
 {
     const dim3 G(grid), B(kBlock);
     if (gt == 2) {
-        launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 2>, G, B, lds, a);
+        // 8 entries and the node's values in flight up to one and a half tiles
+        // per CU (FP64: 158 tiles 9.7 against 11.3 us for 4, 351 tiles 11.0 /
+        // 11.4; split FP32 8.7 / 9.8), 4 above (514 tiles 13.7 / 12.7, 1024
+        // 26.7 / 21.5)
+        bool small = false;
+        if constexpr (TL) {
+            small = 2 * c->n_tiles <= 3 * (int64_t)c->cu_count;
+            if (small) launch_k(c, 1, k_rhs_transpose<4, TM, 8, true, 2>, G, B, lds, a);
+        }
+        if (!small) launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 2>, G, B, lds, a);
     } else if (gt == 3) {
         launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 3>, G, B, lds, a);
     } else {
         // entries per batch, two batches in turn; the default: 8 while every
-        // tile has a CU of its own (256^2 nodes: 11.8 against 12.7 us for 4,
-        // split-FP32 9.7 against 11.1), 4 above, where 8 costs resident
-        // workgroups (512^2: 39.7 against 36.5)
+        // tile has a CU of its own (256^2 nodes: 11.8 against 12.5 us for 4,
+        // split-FP32 10.0 against 11.4), 4 above, where 8 costs resident
+        // workgroups (300^2: 15.1 against 14.5, 363^2: 24.3 / 18.7)
         int bt = c->tune_transpose_batch[TM];
         if (bt == 0 && TL && c->n_tiles <= c->cu_count) bt = 8;
         switch (bt) {
