@@ -2508,7 +2508,8 @@ static void launch_flux_bt(mf_ctx* c, int prec, const RhsArgs& a_in, int hvk, bo
 // Variants compiled per stencil size, by the entries in flight per thread
 // (the tuning value): 3 and 5 are one batch at a time, 6 and 10 two batches
 // of 3 and 5 in turn (the next one in flight while the one at hand is used).
-// The Tominec variants exist for 5 and 10 only.
+// The Tominec variants exist for 5 and 10 only; other values mean the default
+// there.
 // The default (0): up to two tiles per CU the few wavefronts cannot cover
 // each other's memory latency, and two batches in turn are faster; above,
 // their registers cost a resident workgroup.  Stencil kernel (us), one batch
@@ -2516,11 +2517,18 @@ static void launch_flux_bt(mf_ctx* c, int prec, const RhsArgs& a_in, int hvk, bo
 // (two of 5: 13.6), FP64 14.3 / 12.3, with Flyer 13.2 / 11.1, split-FP32
 // 11.6 / 11.1; 300^2 16.7 / 16.8, 16.2 / 15.1, 14.8 / 14.1, 13.4 / 13.6;
 // 512^2 37.3 / 37.4, 39.0 / 40.0, 34.2 / 33.4, 21.7 / 23.5.
+// With the residual viscosity and Tominec in FP64 the three operators' loads
+// outrun one batch: from four tiles per CU two batches of 5 again (one of 5 /
+// two of 5: 512^2 reference order 57.6 / 51.5, FP64 53.5 / 49.4; 724^2 106.0 /
+// 105.0, 104.8 / 99.0; but 363^2 28.3 / 32.5, 24.9 / 27.3, and split FP32 at
+// 512^2 27.7 / 31.6; without the viscosity 44.3 / 44.7, 39.9 / 37.9).
 template <int V>
 static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool rv, unsigned grid)
 {
     int bt = c->tune_flux_batch[prec];
     const bool tl = c->tiles_a && !c->tm_dirty;
+    if ((hvk & 2) && bt != 5 && bt != 10) bt = 0;
+    if (bt == 0 && tl && hvk >= 2 && rv && prec != MF_PREC_SPLIT32 && c->k == 30 && c->n_tiles >= 4 * c->cu_count) bt = 10;
     if (bt == 0 && tl && c->n_tiles <= c->cu_count) bt = prec == MF_PREC_F64_REF || c->k != 30 ? 10 : 6;
     if (bt == 0 && tl && c->n_tiles <= 2 * c->cu_count && c->k == 30) bt = 6;
     switch (c->k) {
@@ -2533,7 +2541,7 @@ static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool r
             else launch_flux_bt<V, 20, 5, false>(c, prec, a, hvk, rv, grid);
             break;
         case 30:
-            if (hvk & 2) bt = bt == 6 || bt == 10 ? 10 : 0;
+            if ((hvk & 2) && bt == 6) bt = 10;
             if (bt == 3) launch_flux_bt<V, 30, 3, false>(c, prec, a, hvk, rv, grid);
             else if (bt == 6) launch_flux_bt<V, 30, 3, true>(c, prec, a, hvk, rv, grid);
             else if (bt == 10) launch_flux_bt<V, 30, 5, true>(c, prec, a, hvk, rv, grid);
