@@ -828,11 +828,11 @@ int mf_weights_ragged_get(mf_ctx* c, double* wx, double* wy)
 
 // The stored FSAL stage as it was before its next boundary pass (which the
 // step that wrote it applied): before the boundary conditions change, or for
-// steps that run that pass themselves.  With the residual viscosity the
-// stage stays as it is (its sums go with it).
+// steps that run that pass themselves.  The next resumed step then takes it
+// as a raw state (see ssprk_step).
 static int raw_fsal(mf_ctx* c)
 {
-    if (!c->fsal_valid || !c->fsal_handed || c->fsal_sums) return MF_OK;
+    if (!c->fsal_valid || !c->fsal_handed) return MF_OK;
     c->fsal_handed = false;
     return c->d_sraw ? run_restore_raw(c, c->d_S) : MF_OK;
 }
@@ -1350,10 +1350,12 @@ static bool stage_handover(const mf_ctx* c, bool limiter)
 // With hand, every rhs! of the step takes its input with its first boundary
 // pass (and sums) from the rhs! before it and leaves the same for the next:
 // T's and U's at this step's stage times t + dt/2 and t + dt, S's at the
-// next step's t_next + dt.  The time moves on in the stage kernels: the
+// next step's t_next + dt.  With raw_s the stored S has had neither (the
+// boundary conditions changed since it was written, or the call that wrote it
+// did not hand over): its rhs! runs the pass and the sums itself.  The time moves on in the stage kernels: the
 // second stage writes t_next = t + dt, the last makes it t (with the history
 // callback, which needs both, the callback does).
-static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history, bool hand)
+static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history, bool hand, bool raw_s = false)
 {
     int rc;
     auto limit = [&](double* u) -> int {
@@ -1367,7 +1369,8 @@ static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history
     s2.dt = dt;
     s2.uprev = U;
     s2.out = c->d_T;
-    s2.handed_in = s2.handed_out = hand;
+    s2.handed_in = hand && !raw_s;
+    s2.handed_out = hand;
     s2.out_dt_off = dt / 2.0;
     s2.time = StageOut::kTimeNext;
     s2.u_dead = true;
@@ -1408,14 +1411,15 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
     const bool residual = c->visc_mode == MF_VISC_RESIDUAL;
     const bool history = (flags & MF_STEP_HISTORY) && residual;
     const bool hand = stage_handover(c, limiter);
-    if (hand && !residual && c->have_bc && !c->d_sraw &&
+    if (hand && c->have_bc && !c->d_sraw &&
         (rc = dalloc(c, &c->d_sraw, (size_t)c->bc.nb * kMaxVar)))
         return rc;
+    bool raw_s = false;
     if (resume) {
         if (!c->fsal_valid || c->fsal_dt != dt)
             return fail(c, MF_ERR_STATE, "mf_ssprk33: resume needs the previous call's state and the same dt");
-        // with the residual viscosity the stored FSAL stage carries the
-        // next boundary pass and sums exactly when no stage limiter runs
+        // with the residual viscosity the stage of a call without a stage
+        // limiter is resumed without one only, and the other way round
         if (c->fsal_sums != (hand && residual))
             return fail(c, MF_ERR_STATE,
                         "mf_ssprk33: resume needs the previous call's stage limiter and viscosity settings");
@@ -1424,7 +1428,7 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
             return MF_OK;
         }
         if (!hand && (rc = raw_fsal(c))) return rc;
-        if (hand && !c->fsal_handed && (rc = bc_pass_state(c, c->d_S, dt))) return rc;
+        raw_s = hand && !c->fsal_handed;
     } else {
         if ((rc = run_set_time(c, t0, 0))) return rc;
         if (history && (rc = run_history(c, c->d_buf[MF_BUF_U], 1))) return rc;
@@ -1438,6 +1442,9 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
         if ((rc = run_rhs(c, precision, c->d_buf[MF_BUF_U], c->d_buf[MF_BUF_DU], 0.0, s1))) return rc;
         c->host_success_iter = 0;
     }
+    int n = 0;
+    if (raw_s && (rc = ssprk_step(c, dt, precision, limiter, history, hand, true))) return rc;
+    if (raw_s) n = 1;
     if (flags & MF_STEP_GRAPH) {
         // every step reads its time from device memory, so a graph of
         // several consecutive steps replays like the same steps one by one
@@ -1469,11 +1476,10 @@ int mf_ssprk33(mf_ctx* c, double t0, double dt, int n_steps, int precision, int 
         if (n_steps >= kGraphSteps && !c->multi_exec &&
             (rc = capture(kGraphSteps, &c->multi_graph, &c->multi_exec)))
             return rc;
-        int n = 0;
         for (; n + kGraphSteps <= n_steps; n += kGraphSteps) MF_HIP(c, hipGraphLaunch(c->multi_exec, c->stream));
         for (; n < n_steps; ++n) MF_HIP(c, hipGraphLaunch(c->step_exec, c->stream));
     } else {
-        for (int n = 0; n < n_steps; ++n)
+        for (; n < n_steps; ++n)
             if ((rc = ssprk_step(c, dt, precision, limiter, history, hand))) return rc;
     }
     c->fsal_dt = dt;
