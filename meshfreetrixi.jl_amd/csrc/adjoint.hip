@@ -395,11 +395,12 @@ int mf_rhs_vjp(mf_ctx* c, double t)
         return fail(c, MF_ERR_UNSUPPORTED, "mf_rhs_vjp: sources have no adjoint in this build");
     if ((rc = prepare_vjp(c))) return rc;
     const HostTime time(c, t);
-    // J is evaluated at P u: boundary pass on a copy of u
-    if ((rc = copy_state(c, c->d_S, c->d_buf[MF_BUF_U]))) return rc;
-    if ((rc = bc_pass_state(c, c->d_S, 0.0))) return rc;
+    // J is evaluated at P u: boundary pass on a copy of u (in T, which holds
+    // nothing between calls; S may be the stage that a resumed step starts from)
+    if ((rc = copy_state(c, c->d_T, c->d_buf[MF_BUF_U]))) return rc;
+    if ((rc = bc_pass_state(c, c->d_T, 0.0))) return rc;
     VjpArgs a = vjp_args(c);
-    a.x = c->d_S;
+    a.x = c->d_T;
     a.lam = c->d_buf[MF_BUF_AUX0];
     a.out = c->d_buf[MF_BUF_AUX1];
     if ((rc = launch_vjp(c, a))) return rc;

@@ -77,3 +77,22 @@ def test_boundary_changes_between_resumed_calls(residual, change):
         for a, b in zip(out[mode], out[GENERAL]):
             assert np.isfinite(a).all()
             assert np.abs(a - b).max() <= (1e-10 * np.abs(b).max() if residual else 0.0)
+
+
+@pytest.mark.parametrize("table", [False, True])
+def test_adjoint_between_resumed_calls(table):
+    """mf_rhs_vjp leaves the state and the stored stage alone, also when the
+    boundary values change after it: the same bits as without it."""
+    ctx, u0, boundary = euler(False, table)
+    ctx.upload(L.MF_BUF_AUX0, np.ascontiguousarray(u0[::-1]))
+    out = []
+    for vjp in (False, True):
+        boundary(1.0)
+        ctx.upload(L.MF_BUF_U, u0)
+        ctx.ssprk33(0.0, DT, 2, L.MF_PREC_F64, 0)
+        if vjp:
+            ctx.rhs_vjp(2 * DT)
+        boundary(1.01)
+        ctx.ssprk33(2 * DT, DT, 3, L.MF_PREC_F64, 0, resume=True)
+        out.append(ctx.download(L.MF_BUF_U))
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
