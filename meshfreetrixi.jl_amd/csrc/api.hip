@@ -1312,6 +1312,7 @@ int mf_limiter_zhang_shu(mf_ctx* c, double threshold, int variable)
     if (variable != MF_VAR_DENSITY && variable != MF_VAR_PRESSURE) return fail(c, MF_ERR_ARGUMENT, "limiter: bad variable");
     if (variable == MF_VAR_PRESSURE && c->nvar != 4) return fail(c, MF_ERR_UNSUPPORTED, "limiter: pressure needs Euler");
     if ((rc = ensure_state(c))) return rc;
+    c->fsal_valid = false;  // the stored stage belongs to u as it was
     if ((rc = run_limiter(c, c->d_buf[MF_BUF_U], 1, &threshold, &variable))) return rc;
     MF_HIP(c, hipStreamSynchronize(c->stream));
     return MF_OK;

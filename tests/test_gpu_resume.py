@@ -96,3 +96,21 @@ def test_adjoint_between_resumed_calls(table):
         ctx.ssprk33(2 * DT, DT, 3, L.MF_PREC_F64, 0, resume=True)
         out.append(ctx.download(L.MF_BUF_U))
     assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
+
+
+def test_limiter_ends_a_resumable_integration():
+    """mf_limiter_zhang_shu changes the state that the stored stage was formed
+    from, as an upload does: the next call starts anew or is an error."""
+    ctx, u0, _ = euler(False)
+    ctx.upload(L.MF_BUF_U, u0)
+    ctx.ssprk33(0.0, DT, 2, L.MF_PREC_F64, 0)
+    ctx.limiter_zhang_shu(float(ctx.download(L.MF_BUF_U)[0].mean()), L.MF_VAR_DENSITY)
+    u = ctx.download(L.MF_BUF_U)
+    with pytest.raises(L.MfError) as e:
+        ctx.ssprk33(2 * DT, DT, 1, L.MF_PREC_F64, 0, resume=True)
+    assert e.value.code == L.MF_ERR_STATE
+    ctx.ssprk33(2 * DT, DT, 1, L.MF_PREC_F64, 0)
+    got = ctx.download(L.MF_BUF_U)
+    ctx.upload(L.MF_BUF_U, u)
+    ctx.ssprk33(2 * DT, DT, 1, L.MF_PREC_F64, 0)
+    assert np.isfinite(got).all() and np.array_equal(got, ctx.download(L.MF_BUF_U))
