@@ -638,22 +638,32 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
+    auto entry = [&](int s, int32_t& j, double2& w, double& hw, double& lw) {
+        if constexpr (TL)
+            j = entry_of<TL>(a.la, blk, K, s, N, i);
+        else
+            j = entry_of<TL>(a.idx, blk, K, s, N, i);
+        w = entry_of<TL>(a.wxy, blk, K, s, N, i);
+        if constexpr (FLY) hw = entry_of<TL>(a.hv, blk, K, s, N, i);
+        if constexpr (TOM) lw = entry_of<TL>(a.lap, blk, K, s, N, i);
+    };
     auto load = [&](int s0, FluxBatch<double2, double, BT>& q) {
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
-            const int s = s0 + b;
-            if ((NS && NS % BT == 0) || s < K) {
-                if constexpr (TL)
-                    q.j[b] = entry_of<TL>(a.la, blk, K, s, N, i);
-                else
-                    q.j[b] = entry_of<TL>(a.idx, blk, K, s, N, i);
-                q.w[b] = entry_of<TL>(a.wxy, blk, K, s, N, i);
-                if constexpr (FLY) q.hw[b] = entry_of<TL>(a.hv, blk, K, s, N, i);
-                if constexpr (TOM) q.lw[b] = entry_of<TL>(a.lap, blk, K, s, N, i);
+            if constexpr (NS && NS % BT == 0) {
+                entry(s0 + b, q.j[b], q.w[b], q.hw[b], q.lw[b]);
             } else {
-                q.j[b] = TL ? 0 : (int32_t)i;
-                q.w[b] = make_double2(0.0, 0.0);
-                q.hw[b] = q.lw[b] = 0.0;
+                // into locals first: stored into the batch from both branches, the
+                // batch stayed in scratch memory (K = 25, 600^2 nodes: 42.3 us,
+                // with the locals 31.2)
+                int32_t j = TL ? 0 : (int32_t)i;
+                double2 w = make_double2(0.0, 0.0);
+                double hw = 0.0, lw = 0.0;
+                if (s0 + b < K) entry(s0 + b, j, w, hw, lw);
+                q.j[b] = j;
+                q.w[b] = w;
+                if constexpr (FLY) q.hw[b] = hw;
+                if constexpr (TOM) q.lw[b] = lw;
             }
         }
     };
@@ -922,24 +932,32 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
     double pm[4] = {-1.0, -1.0, -1.0, -1.0};
     const bool rvres = RV && a.visc == MF_VISC_RESIDUAL;
     if (rvres) prefetch_max_partials(a, pm);
+    auto entry = [&](int s, int32_t& j, float2& w, float& hw, float& lw) {
+        if constexpr (TL)
+            j = entry_of<TL>(a.la, blk, K, s, N, i);
+        else if constexpr (D16)
+            j = (int32_t)i + (int32_t)entry_of<TL>(a.didx, blk, K, s, N, i);
+        else
+            j = entry_of<TL>(a.idx, blk, K, s, N, i);
+        w = entry_of<TL>(a.wxy32, blk, K, s, N, i);
+        if constexpr (FLY) hw = entry_of<TL>(a.hv32, blk, K, s, N, i);
+        if constexpr (TOM) lw = entry_of<TL>(a.lap32, blk, K, s, N, i);
+    };
     auto load = [&](int s0, FluxBatch<float2, float, BT>& q) {
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
-            const int s = s0 + b;
-            if ((NS && NS % BT == 0) || s < K) {
-                if constexpr (TL)
-                    q.j[b] = entry_of<TL>(a.la, blk, K, s, N, i);
-                else if constexpr (D16)
-                    q.j[b] = (int32_t)i + (int32_t)entry_of<TL>(a.didx, blk, K, s, N, i);
-                else
-                    q.j[b] = entry_of<TL>(a.idx, blk, K, s, N, i);
-                q.w[b] = entry_of<TL>(a.wxy32, blk, K, s, N, i);
-                if constexpr (FLY) q.hw[b] = entry_of<TL>(a.hv32, blk, K, s, N, i);
-                if constexpr (TOM) q.lw[b] = entry_of<TL>(a.lap32, blk, K, s, N, i);
+            if constexpr (NS && NS % BT == 0) {
+                entry(s0 + b, q.j[b], q.w[b], q.hw[b], q.lw[b]);
             } else {
-                q.j[b] = TL ? 0 : (int32_t)i;
-                q.w[b] = make_float2(0.0f, 0.0f);
-                q.hw[b] = q.lw[b] = 0.0f;
+                // into locals first, as in k_rhs_f64
+                int32_t j = TL ? 0 : (int32_t)i;
+                float2 w = make_float2(0.0f, 0.0f);
+                float hw = 0.0f, lw = 0.0f;
+                if (s0 + b < K) entry(s0 + b, j, w, hw, lw);
+                q.j[b] = j;
+                q.w[b] = w;
+                if constexpr (FLY) q.hw[b] = hw;
+                if constexpr (TOM) q.lw[b] = lw;
             }
         }
     };
