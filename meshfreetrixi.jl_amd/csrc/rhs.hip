@@ -579,6 +579,31 @@ __device__ __forceinline__ T entry_of(const T* p, int64_t blk, int K, int s, int
         return p[(int64_t)s * N + i];
 }
 
+// Whether the stencil kernels with a viscosity load the node's state and
+// approx_du before the row's entries.  With Flyer or Tominec and one batch at a
+// time the registers held through the sums cost the reference order a wavefront
+// per SIMD (126 -> 146 VGPRs; residual viscosity, K = 20, 512^2 nodes: with
+// Flyer 38.4 us, loaded late 35.1, with Tominec 43.4 / 37.0) and FP64 as much for
+// stencil sizes without a variant of their own (K = 25, Tominec, 512^2 51.7 /
+// 47.6); FP64 with one is faster with the values held (K = 30, Flyer, 600^2 72.2 /
+// 81.8).
+template <bool F64, int NS, int HVK, bool PF>
+__device__ constexpr bool hold_node()
+{
+    return PF || HVK == 0 || (F64 && NS);
+}
+
+// Wavefronts per SIMD that k_rhs_f64 is compiled for at least: five for batches
+// of 5 without a viscosity (left to itself the compiler takes 104 to 126 VGPRs,
+// four wavefronts, and from four to five tiles per CU the last workgroups wait
+// for a second round).  No source, K = 30, 540^2 nodes 29.9 -> 27.6 us, K = 20,
+// 400^2 13.1 -> 12.3; with Flyer, K = 20, 600^2 34.4 -> 31.0.
+template <int V, int HVK, bool RV, int BT, bool PF, bool TL>
+__device__ constexpr int f64_waves()
+{
+    return V == 4 && TL && !PF && BT == 5 && HVK < 3 && !RV ? 5 : 1;
+}
+
 // One batch of stencil entries of a row: halo positions or nodes, (Dx, Dy)
 // (or one of them), Flyer and Laplacian weights.
 template <class W, class W1, int BT>
@@ -621,7 +646,7 @@ __device__ __forceinline__ void for_batches(int K, Q& q0, Load load, Use use)
 // with weight 0.  TL: neighbour records come from the LDS halo, addressed
 // by 16-bit halo positions (same slot-major layout as idx).
 template <int V, int NS, int HVK, bool RV, int BT, bool PF, bool TL>
-__global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
+__global__ __launch_bounds__(kBlock, (f64_waves<V, HVK, RV, BT, PF, TL>())) void k_rhs_f64(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
@@ -673,10 +698,11 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
     stage_halo_a<V, TL>(a, blk, lds, rvres, pm, wmax);
     if (!rvres && !live) return;
     double ui[V], ad[V];  // the node's state and approx_du, in flight through the loop
-    if constexpr (RV) {
+    auto load_node = [&] {
         load_state<V>(a.u, i, ui);
         if (rvres) load_state<V>(a.approx, i, ad);
-    }
+    };
+    if constexpr (RV && hold_node<true, NS, HVK, PF>()) load_node();
     double ax[V], ay[V], gx[V], gy[V], hh[V], ll[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) ax[v] = ay[v] = gx[v] = gy[v] = hh[v] = ll[v] = 0.0;
@@ -726,6 +752,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_f64(const RhsArgs a)
         if constexpr (RV) {
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
+            if constexpr (!hold_node<true, NS, HVK, PF>()) load_node();
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, ui, du, ad, ninf, &code);
@@ -868,10 +895,11 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
     if constexpr (!RV && !TOM) load_tail(a, i, tail);
     ref_pass<V, NS, RV, BT, PF, 0, TL>(a, blk, i, K, du, gx, lds, a.wx_s, q0, a.wy_s);
     double ui[V], ad[V];  // the node's state and approx_du, in flight through the y pass
-    if constexpr (RV) {
+    auto load_node = [&] {
         load_state<V>(a.u, i, ui);
         if (rvres) load_state<V>(a.approx, i, ad);
-    }
+    };
+    if constexpr (RV && hold_node<false, NS, HVK, PF>()) load_node();
     const bool fly = FLY && a.flyer_a;
     ref_pass<V, NS, RV, BT, PF, 1, TL>(a, blk, i, K, du, gy, lds, a.wy_s, q0, fly ? a.hv_s : (TOM ? a.lap_s : nullptr));
     if constexpr (FLY) {
@@ -881,6 +909,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
         if constexpr (RV) {
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
+            if constexpr (!hold_node<false, NS, HVK, PF>()) load_node();
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, ui, du, ad, ninf, &code);
@@ -965,9 +994,10 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
     if constexpr (PF) load(0, q0);
     double ui[V], fi1[V], fi2[V], ad[V];
     load_state<V>(a.u, i, ui);
-    if constexpr (RV) {
+    auto load_node = [&] {
         if (rvres) load_state<V>(a.approx, i, ad);
-    }
+    };
+    if constexpr (RV && hold_node<false, NS, HVK, PF>()) load_node();
     __shared__ double wmax[kBlock / 64][4];
     stage_halo_a<V, TL>(a, blk, lds, rvres, pm, wmax);
     if (!rvres && !live) return;
@@ -1033,6 +1063,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
         if constexpr (RV) {
             int8_t code = 1;
             double ninf[4] = {1.0, 1.0, 1.0, 1.0};
+            if constexpr (!hold_node<false, NS, HVK, PF>()) load_node();
             if (rvres) finish_norms<TL>(a, pm, wmax, ninf);
             if (!live) return;
             const double e = node_viscosity(a, ui, du, ad, ninf, &code);
