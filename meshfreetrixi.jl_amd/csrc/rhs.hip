@@ -195,6 +195,8 @@ struct RhsArgs {
     int* tm_iter;
 };
 
+// By thread 0 of block 0, which has a node in every kernel (the transposed
+// tiles sort their rows longest first, rows past the last node at the end).
 __device__ __forceinline__ void move_time(const RhsArgs& a)
 {
     if (a.tm_dst && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -340,6 +342,9 @@ __device__ __forceinline__ void emit(const RhsArgs& a, int64_t i, const NodeTail
         store_state<V>(a.du, i, du);
         return;
     }
+    // here and not at the start of the kernel, where every block waited for
+    // the arguments that move_time reads (0.3 us a launch)
+    move_time(a);
     stage_value(a, i, t, du, o);
     if (a.obc.flag) {
         int32_t e;
@@ -650,7 +655,6 @@ __global__ __launch_bounds__(kBlock, (f64_waves<V, HVK, RV, BT, PF, TL>())) void
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
-    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int64_t N = a.N;
@@ -871,7 +875,6 @@ __global__ __launch_bounds__(kBlock) void k_rhs_ref(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
-    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int K = NS ? NS : a.k;
@@ -948,7 +951,6 @@ __global__ __launch_bounds__(kBlock) void k_rhs_s32(const RhsArgs a)
 {
     constexpr bool FLY = HVK & 1, TOM = HVK & 2;
     extern __shared__ double lds[];
-    if constexpr (!RV && !TOM) move_time(a);  // phase A writes no stage
     const int64_t blk = remapped_block();
     if (blk * kBlock >= a.N) return;  // whole block
     const int64_t N = a.N;
@@ -1128,7 +1130,6 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
     constexpr int RU = (HG ? 2 : 0) + (HL ? 1 : 0);  // V-value units per halo record
     constexpr int LU = HG ? 2 : 0;                   // unit of L in a record
     extern __shared__ double lds[];
-    move_time(a);
     int64_t i, off = 0;
     int W = 0;
     const int lane = threadIdx.x & 63;
@@ -2254,7 +2255,6 @@ template <bool TL>
 __global__ __launch_bounds__(kBlock) void k_igr_apply(const IgrArgs g, const RhsArgs a)
 {
     extern __shared__ double lds[];
-    move_time(a);
     const int64_t lb = remapped_block();
     if (lb >= g.nblk) return;  // whole block
     const int64_t i = lb * kBlock + threadIdx.x;
