@@ -313,9 +313,15 @@ __device__ __forceinline__ int64_t lds_chunk(int64_t q, int c)
 
 // The nh halo entries of a tile by the block's threads, R per thread and trip:
 // the R node ids load together, then what get reads of the nodes, then put
-// stores it.  One entry per trip cost two dependent loads for each 256 entries
-// (rhs! with residual viscosity, split FP32, 131,769 nodes: 59.7 -> 57.5 us).
-constexpr int kHaloLoads = 2;  // a halo is 1.4 to 2 times its tile's nodes
+// stores it.  One entry per trip cost two dependent loads for each 256 entries.
+// The empty asm keeps the loads ahead of the first put: without it the compiler
+// moves those of the second entry under put's condition, after the first put
+// (stencil kernel, FP64, K = 20, no source: 128^2 nodes 6.1 -> 5.2 us, 256^2 6.5
+// -> 6.0, 512^2 18.1 -> 17.0).
+// Two entries per thread and trip: the halos of Morton-ordered clouds measured
+// 1.4 to 2 times their tile's nodes for K of 15 to 30.  Larger ones, up to what
+// LDS holds, take more trips.
+constexpr int kHaloLoads = 2;
 
 template <int R, class T, class Get, class Put>
 __device__ __forceinline__ void for_halo(int nh, const int32_t* __restrict__ ids, Get get, Put put)
@@ -327,6 +333,7 @@ __device__ __forceinline__ void for_halo(int nh, const int32_t* __restrict__ ids
         for (int r = 0; r < R; ++r) j[r] = ids[min(q0 + r * kBlock, nh - 1)];
 #pragma unroll
         for (int r = 0; r < R; ++r) get(j[r], v[r]);
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int r = 0; r < R; ++r)
             if (q0 + r * kBlock < nh) put(q0 + r * kBlock, v[r]);
