@@ -714,6 +714,10 @@ __global__ __launch_bounds__(kBlock, (f64_waves<V, HVK, RV, BT, PF, TL>())) void
         double uj[BT][TL ? rec_len<V>() : V];
 #pragma unroll
         for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, q.j[b], uj[b]);
+        // the whole batch's gathers from global memory in flight before the
+        // first is used; the scheduler otherwise waits for one after another
+        // (256^2 nodes, K = 30, no tiles: 17.1 -> 10.7 us)
+        if constexpr (!TL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             double f1[V], f2[V];
@@ -825,6 +829,7 @@ __device__ __forceinline__ void ref_pass(const RhsArgs& a, int64_t blk, int64_t 
         double uj[BT][TL ? rec_len<V>() : V];
 #pragma unroll
         for (int b = 0; b < BT; ++b) load_nb<V, TL>(a, lds, q.j[b], uj[b]);
+        if constexpr (!TL) __builtin_amdgcn_sched_barrier(0);  // as in k_rhs_f64
 #pragma unroll
         for (int b = 0; b < BT; ++b) {
             if (!((NS && NS % BT == 0) || s0 + b < K)) continue;
@@ -1221,7 +1226,6 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             const int64_t slice = i >> 6;
             off = a.sell_off[slice];
             W = a.sell_w[slice];
-            if (W > 0) load(0, q0);  // a slice of nodes that no stencil names has no entries
         }
     }
     constexpr bool kAhead = TL && BT > 4;  // see NodeTail
@@ -1300,14 +1304,25 @@ __global__ __launch_bounds__(kBlock) void k_rhs_transpose(const RhsArgs a)
             }
         }
     };
+    if constexpr (TL) {
 #pragma unroll 1
-    for (int e0 = 0; e0 < W; e0 += 2 * BT) {
-        if (e0 + BT < W) load(e0 + BT, q1);
-        __builtin_amdgcn_sched_barrier(0);
-        use(e0, q0);
-        if (e0 + 2 * BT < W) load(e0 + 2 * BT, q0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (e0 + BT < W) use(e0 + BT, q1);
+        for (int e0 = 0; e0 < W; e0 += 2 * BT) {
+            if (e0 + BT < W) load(e0 + BT, q1);
+            __builtin_amdgcn_sched_barrier(0);
+            use(e0, q0);
+            if (e0 + 2 * BT < W) load(e0 + 2 * BT, q0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (e0 + BT < W) use(e0 + BT, q1);
+        }
+    } else {
+        // one batch at a time: a batch's gathers from global memory fill the
+        // registers already (a second batch: 92 -> 132 VGPRs; 512^2 nodes, K = 20,
+        // Tominec 20.7 -> 25.5 us)
+#pragma unroll 1
+        for (int e0 = 0; e0 < W; e0 += BT) {
+            load(e0, q0);
+            use(e0, q0);
+        }
     }
     double o[4] = {0.0, 0.0, 0.0, 0.0};  // the stored output (staged stages)
     if (live) {

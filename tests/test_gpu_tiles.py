@@ -159,3 +159,32 @@ def test_slices_that_no_stencil_names(n, unnamed):
     operators(ctx, idx, rng)
     both_ways(ctx, n, rng)
     assert ctx.tile_info()["tiles_a"] == 0  # the last pass was the one without
+
+
+def test_transposed_halos_that_do_not_fit():
+    """Stencils of 64 nodes: the stencil halos fit (1,024 records), the transposed
+    ones of G and L together (682) do not: tiled stencil kernel, global
+    transposed gather."""
+    rng = np.random.default_rng(11)
+    x, y, _, _, _ = cloud_square(61, 151)
+    n = len(x)
+    ctx = L.Context(0)
+    ctx.set_equations(L.MF_EQ_EULER_2D, 1.4)
+    ctx.set_points(x, y)
+    idx = ctx.knn(64)[0]
+    operators(ctx, idx, rng)
+    ctx.set_operator(L.MF_OP_LAPLACIAN, rng.standard_normal(idx.shape))
+    ctx.set_source_hyperviscosity_tominec(1e-3)
+    ctx.set_source_viscosity(L.MF_VISC_UPWIND, 1.0, 1.0, 0.01, 3, True)
+    ctx.set_source_order([L.MF_SRC_VISCOSITY, L.MF_SRC_TOMINEC])
+    u0 = np.ascontiguousarray(np.stack([1.0 + 0.1 * rng.random(n), rng.standard_normal(n), rng.standard_normal(n),
+                                        5.0 + rng.random(n)]))
+    for prec in (L.MF_PREC_F64, L.MF_PREC_F64_REF, L.MF_PREC_SPLIT32):
+        out = []
+        for tiles in (1, 0):
+            ctx.set_tuning(L.MF_TUNE_TILES, tiles)
+            u, du = u0.copy(), np.empty_like(u0)
+            ctx.rhs_host(0.0, u, du, prec)
+            assert (ctx.tile_info()["tiles_a"], ctx.tile_info()["tiles_b"]) == (tiles, 0)
+            out.append(du)
+        assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
