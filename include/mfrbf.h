@@ -357,8 +357,14 @@ int mf_ssprk33_vjp(mf_ctx* ctx, double t0, double dt, int n_steps, int checkpoin
 /* ------------------------------------------------------------- tuning */
 #define MF_TUNE_FLUX_BATCH 0      /* stencil entries in flight per thread: 3, 5 (one batch at a time), 6,
                                      10 (two batches of 3, 5 in turn); 0 (default): by the number of
-                                     LDS tiles per compute unit */
-#define MF_TUNE_TRANSPOSE_BATCH 1 /* transposed entries per batch, two batches in turn: 2, 4, 8; 0
+                                     LDS tiles per compute unit, the sources and the precision.  All
+                                     four for stencils of 30 nodes; 15 and 20 nodes have 5 and 10 (3
+                                     and 6 mean 5 there), other sizes one batch of 4 whatever the
+                                     value; with a Tominec source 3 and 6 mean 0, and without tiles 6
+                                     and 10 mean 3 and 5 */
+#define MF_TUNE_TRANSPOSE_BATCH 1 /* transposed entries per batch, two batches in turn (one without
+                                     tiles): 2, 4, 8 with a viscosity; with a Tominec source alone 8
+                                     (with tiles) and else 4, with both 2 (with tiles) and else 4; 0
                                      (default): by the number of LDS tiles per compute unit */
 #define MF_TUNE_NODE_ORDER 2      /* internal node order for the next mf_set_points: 0 Morton
                                      (default), 1 the caller's order; precision is ignored */
@@ -372,8 +378,8 @@ int mf_ssprk33_vjp(mf_ctx* ctx, double t0, double dt, int n_steps, int checkpoin
                                      and stencils have at least twice as many nodes as
                                      monomials); precision is ignored */
 /* Selects a compiled kernel variant for one precision (MF_PREC_*, or -1 for
- * all).  A batch size that does not divide the stencil size falls back to
- * the default.  Results do not depend on it (the per-node operation order is
+ * all).  Values are accepted for every stencil size; which variant they mean
+ * is said at each key.  Results do not depend on it (the per-node operation order is
  * the same for every batch size).  No counterpart in the reference (the CPU
  * path has no launch shapes); set by the autotuner of the Python package. */
 int mf_set_tuning(mf_ctx* ctx, int key, int precision, int value);

@@ -2572,29 +2572,49 @@ static void launch_flux_bt(mf_ctx* c, int prec, const RhsArgs& a_in, int hvk, bo
 // Variants compiled per stencil size, by the entries in flight per thread
 // (the tuning value): 3 and 5 are one batch at a time, 6 and 10 two batches
 // of 3 and 5 in turn (the next one in flight while the one at hand is used).
-// The Tominec variants exist for 5 and 10 only; other values mean the default
-// there.
-// The default (0): up to two tiles per CU the few wavefronts cannot cover
-// each other's memory latency, and two batches in turn are faster; above,
-// their registers cost a resident workgroup.  Stencil kernel (us), one batch
-// of 5 / two of 3: 256^2 nodes (one tile per CU) reference order 14.6 / 14.4
-// (two of 5: 13.6), FP64 14.3 / 12.3, with Flyer 13.2 / 11.1, split-FP32
-// 11.6 / 11.1; 300^2 16.7 / 16.8, 16.2 / 15.1, 14.8 / 14.1, 13.4 / 13.6;
-// 512^2 37.3 / 37.4, 39.0 / 40.0, 34.2 / 33.4, 21.7 / 23.5.
-// With the residual viscosity and Tominec in FP64 the three operators' loads
-// outrun one batch: from four tiles per CU two batches of 5 again (one of 5 /
-// two of 5: 512^2 reference order 57.6 / 51.5, FP64 53.5 / 49.4; 724^2 106.0 /
-// 105.0, 104.8 / 99.0; but 363^2 28.3 / 32.5, 24.9 / 27.3, and split FP32 at
-// 512^2 27.7 / 31.6; without the viscosity 44.3 / 44.7, 39.9 / 37.9).
+// K = 15 and 20 have 5 and 10, K = 30 all four; the Tominec variants exist for
+// 5 and 10.  Other K run one batch of 4.  Without tiles there is one batch.
+//
+// The default with tiles.  Up to one tile per CU the few wavefronts cannot
+// cover each other's latency and two batches in turn are faster wherever there
+// is more to load than one operator, or a stage to write (the node's values are
+// then loaded ahead, NodeTail); on larger grids their registers cost resident
+// workgroups.  Stencil kernel (us), 5 / 6 / 10 (K = 20: 5 / 10):
+//   no source    FP64        split FP32        reference order
+//   256^2 K=20   6.0 / 6.3   6.6 / 6.9         8.4 / 8.2
+//   256^2 K=30   8.9/9.4/9.6 8.3/8.1/8.5       12.1/11.7/11.3
+//   300^2 K=30   11.7/12.1   11.6/11.7         17.0/16.8
+//   Flyer
+//   256^2 K=20   9.2 / 8.0   6.8 / 6.8         11.6 / 10.1
+//   256^2 K=30   11.9/10.9   9.0/8.9           14.7/14.0/13.3
+//   300^2 K=30   14.3/13.9   12.2/12.2         20.6/19.9
+//   residual viscosity
+//   256^2 K=20   11.9 / 10.9 9.4 / 9.4         11.9 / 11.6
+//   256^2 K=30   14.2/12.0   11.1/11.2         13.9/14.0/13.4
+//   300^2 K=30   16.0/14.5   13.4/13.7         15.9/16.4
+// With Tominec split FP32 is the exception below (256^2, K = 30 with the
+// residual viscosity 11.5 / 12.4), and in FP64 with a viscosity from four tiles
+// per CU the three operators' loads outrun one batch (5 / 10: 512^2 K = 30 52.6 /
+// 48.9, K = 20 36.1 / 34.6; reference order 48.4 / 50.3).  Between: one batch
+// (363^2, K = 20, residual viscosity 16.1 / 19.8).
+static int default_flux_batch(const mf_ctx* c, int prec, int hvk, bool rv, bool stage)
+{
+    const bool f64 = prec == MF_PREC_F64, ref = prec == MF_PREC_F64_REF, more = hvk || rv || stage;
+    if (c->n_tiles <= c->cu_count) {
+        if (c->k == 30) return ref ? 10 : f64 ? (more ? 6 : 5) : ((hvk & 2) ? 5 : 6);
+        return ref || (f64 && more) || stage ? 10 : 5;
+    }
+    if (f64 && rv && (hvk & 2) && c->n_tiles >= 4 * c->cu_count) return 10;
+    if (c->k == 30 && c->n_tiles <= 2 * c->cu_count) return (f64 ? more : ref && more && !rv) ? 6 : 5;
+    return 5;
+}
+
 template <int V>
 static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool rv, unsigned grid)
 {
     int bt = c->tune_flux_batch[prec];
-    const bool tl = c->tiles_a && !c->tm_dirty;
     if ((hvk & 2) && bt != 5 && bt != 10) bt = 0;
-    if (bt == 0 && tl && hvk >= 2 && rv && prec != MF_PREC_SPLIT32 && c->k == 30 && c->n_tiles >= 4 * c->cu_count) bt = 10;
-    if (bt == 0 && tl && c->n_tiles <= c->cu_count) bt = prec == MF_PREC_F64_REF || c->k != 30 ? 10 : 6;
-    if (bt == 0 && tl && c->n_tiles <= 2 * c->cu_count && c->k == 30) bt = 6;
+    if (bt == 0 && c->tiles_a && !c->tm_dirty) bt = default_flux_batch(c, prec, hvk, rv, a.st_kind != ST_NONE);
     switch (c->k) {
         case 15:
             if (bt == 10) launch_flux_bt<V, 15, 5, true>(c, prec, a, hvk, rv, grid);
@@ -2615,8 +2635,12 @@ static void launch_flux_v(mf_ctx* c, int prec, const RhsArgs& a, int hvk, bool r
     }
 }
 
-// gt bit 0: G of the viscosity source, bit 1: L of the Tominec source (its
-// variants take no tuning).
+constexpr size_t kCuLdsBytes = 160 * 1024;
+
+// gt bit 0: G of the viscosity source, bit 1: L of the Tominec source.  The
+// tuning value is the entries per batch, two batches in turn (without tiles
+// one): 2, 4, 8 for G, 4, 8 for L, 2, 4 for both (without tiles 4 there).
+
 template <int TM, bool TL>
 static void launch_transpose_tl(mf_ctx* c, const RhsArgs& a, unsigned grid, size_t lds, int gt)
 {
@@ -2626,13 +2650,23 @@ static void launch_transpose_tl(mf_ctx* c, const RhsArgs& a, unsigned grid, size
         // per CU (FP64: 158 tiles 9.7 against 11.3 us for 4, 351 tiles 11.0 /
         // 11.4; split FP32 8.7 / 9.8), 4 above (514 tiles 13.7 / 12.7, 1024
         // 26.7 / 21.5)
-        bool small = false;
-        if constexpr (TL) {
-            small = 2 * c->n_tiles <= 3 * (int64_t)c->cu_count;
-            if (small) launch_k(c, 1, k_rhs_transpose<4, TM, 8, true, 2>, G, B, lds, a);
-        }
-        if (!small) launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 2>, G, B, lds, a);
+        int bt = c->tune_transpose_batch[TM];
+        if (bt == 0 && 2 * c->n_tiles <= 3 * (int64_t)c->cu_count) bt = 8;
+        if constexpr (TL)
+            if (bt == 8) return launch_k(c, 1, k_rhs_transpose<4, TM, 8, true, 2>, G, B, lds, a);
+        launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 2>, G, B, lds, a);
     } else if (gt == 3) {
+        // batches of 4 hold 164 VGPRs, three workgroups per CU, those of 2 have
+        // 88 to 90: up to three tiles per CU, where LDS lets three workgroups of
+        // FP64 records share a CU, the second round counts (FP64, K = 20: 300^2
+        // nodes 13.7 us against 14.4 for 4, 363^2 18.2 / 20.6, 443^2 22.8 / 23.8,
+        // 512^2 40.1 / 37.9; K = 30 with two workgroups per CU 400^2 39.1 / 37.3;
+        // split FP32, K = 20, 400^2 14.0 / 13.3)
+        int bt = c->tune_transpose_batch[TM];
+        if (bt == 0 && TM != 1 && 3 * lds <= kCuLdsBytes && c->n_tiles > c->cu_count && c->n_tiles <= 3 * c->cu_count)
+            bt = 2;
+        if constexpr (TL)
+            if (bt == 2) return launch_k(c, 1, k_rhs_transpose<4, TM, 2, true, 3>, G, B, lds, a);
         launch_k(c, 1, k_rhs_transpose<4, TM, 4, TL, 3>, G, B, lds, a);
     } else {
         // entries per batch, two batches in turn; the default: 8 while every
@@ -2641,6 +2675,12 @@ static void launch_transpose_tl(mf_ctx* c, const RhsArgs& a, unsigned grid, size
         // workgroups (300^2: 15.1 against 14.5, 363^2: 24.3 / 18.7)
         int bt = c->tune_transpose_batch[TM];
         if (bt == 0 && TL && c->n_tiles <= c->cu_count) bt = 8;
+        // split FP32: five workgroups of batches of 4 share a CU; just above,
+        // where the rest would be a short second round, 2 (eight workgroups:
+        // 600^2, K = 30 27.2 us against 32.5 for 4, 640^2 33.8 / 36.2; 570^2 24.8 /
+        // 23.5, 680^2 50.4 / 42.3)
+        if (bt == 0 && TL && TM == 1 && c->n_tiles > 5 * c->cu_count && 2 * c->n_tiles <= 13 * (int64_t)c->cu_count)
+            bt = 2;
         switch (bt) {
             case 2: launch_k(c, 1, k_rhs_transpose<4, TM, 2, TL, 1>, G, B, lds, a); break;
             case 8: launch_k(c, 1, k_rhs_transpose<4, TM, 8, TL, 1>, G, B, lds, a); break;

@@ -64,3 +64,40 @@ def test_variants_bitwise(sources, k, prec):
                         ref = (u, du)
                     assert np.isfinite(du).all()
                     assert np.array_equal(u, ref[0]) and np.array_equal(du, ref[1]), (side, tiles, fb, tb)
+
+
+@pytest.mark.parametrize("prec", [L.MF_PREC_F64, L.MF_PREC_SPLIT32, L.MF_PREC_F64_REF])
+@pytest.mark.parametrize("side,k", [(8, 15), (17, 20), (33, 30), (33, 23), (321, 20)])
+def test_tominec_transposed_batches(side, k, prec):
+    """The transposed product of the Tominec source alone: each batch by the
+    tuning value, with tiles and without, and the default (side 321: more than
+    one and a half tiles per compute unit)."""
+    ctx, u0 = context(side, k, ("tominec",))
+    out = []
+    for tiles in (0, 1):
+        ctx.set_tuning(L.MF_TUNE_TILES, tiles)
+        for tb in (0, 2, 4, 8):
+            ctx.set_tuning(L.MF_TUNE_TRANSPOSE_BATCH, tb, prec)
+            u, du = u0.copy(), np.empty_like(u0)
+            ctx.rhs_host(0.004, u, du, prec)
+            assert ctx.tile_info()["tiles_b"] == tiles
+            out.append(du)
+    assert np.isfinite(out[0]).all()
+    for du in out[1:]:
+        assert np.array_equal(du, out[0])
+
+
+@pytest.mark.parametrize("prec", [L.MF_PREC_F64, L.MF_PREC_SPLIT32, L.MF_PREC_F64_REF])
+@pytest.mark.parametrize("side,k,sources", [(300, 20, ("residual", "tominec")), (600, 15, ("residual",)),
+                                            (520, 20, ("residual", "tominec")), (300, 30, ("flyer",))])
+def test_default_batches_on_large_clouds(side, k, sources, prec):
+    """The defaults that depend on the tiles per compute unit, against the global
+    gathers."""
+    ctx, u0 = context(side, k, sources)
+    out = []
+    for tiles in (0, 1):
+        ctx.set_tuning(L.MF_TUNE_TILES, tiles)
+        u, du = u0.copy(), np.empty_like(u0)
+        ctx.rhs_host(0.004, u, du, prec)
+        out.append(du)
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
