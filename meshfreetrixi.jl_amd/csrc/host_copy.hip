@@ -11,8 +11,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -22,9 +22,15 @@ namespace mf {
 
 constexpr size_t kChunkBytes = (size_t)2 << 20;
 constexpr int kMaxChunks = 16;              // of the process, whatever its contexts
-constexpr int kCopyThreads = 8;             // per large transfer
+constexpr int kCopyThreads = 8;             // per large transfer, at most one per processor
 constexpr size_t kDirectBytes = (size_t)1 << 20;   // states up to this size: read or written by the kernel
-constexpr size_t kThreadBytes = (size_t)4 << 20;   // transfers from this size: several threads,
+// Transfers by several threads, from these sizes.  To the host they also fault
+// the caller's pages in, which one thread does at about 15 GB/s; towards the
+// device the runtime reads pageable memory at 30 GB/s by itself and the threads
+// gain only once they run for a while (us, runtime / threads, up: 8 MB 268 / 330,
+// 17 MB 502 / 580, 34 MB 982 / 1039, 46 MB 1657 / 1374, 67 MB 2237 / 1900; down: 8
+// MB 489 / 324, 17 MB 942 / 567, 67 MB 3755 / 1852).
+constexpr size_t kThreadBytesUp = (size_t)40 << 20, kThreadBytesDown = (size_t)4 << 20;
 constexpr size_t kGrowBytes = (size_t)8 << 20;     // allocating chunks for them from this size
 
 // The process's pinned chunks: allocated as transfers need them, at most
@@ -142,15 +148,32 @@ static hipError_t copy_chunks(int device, hipStream_t stream, const HostFields& 
     return e;
 }
 
-// The range [d, d + count field_bytes) to or from the fields; complete on
-// return.
+// Whether some field is memory that the runtime knows (pinned, managed): it is
+// copied from or to directly, at the link's rate, which the pinned chunks would
+// only slow down (17 MB 374 us against 573).
+static bool known_memory(const HostFields& f)
+{
+    for (int v = 0; v < f.count; ++v) {
+        hipPointerAttribute_t at;
+        if (hipPointerGetAttributes(&at, f.fields[v]) != hipSuccess)
+            (void)hipGetLastError();
+        else if (at.type != hipMemoryTypeUnregistered)
+            return true;
+    }
+    return false;
+}
+
+// The range [d, d + count field_bytes) to or from the fields; the fields are
+// complete on return, towards the device the stream may still be reading them.
 int copy_fields(mf_ctx* c, void* d, const HostFields& f, bool to_host)
 {
     const size_t bytes = f.field_bytes * (size_t)f.count;
     if (bytes == 0) return MF_OK;
-    const size_t n_chunks = (bytes + kChunkBytes - 1) / kChunkBytes;
-    const Borrowed b(c, bytes >= kThreadBytes ? (int)std::min<size_t>(n_chunks, kCopyThreads) : 0,
-                     bytes >= kGrowBytes);
+    int want = 0;
+    if (bytes >= (to_host ? kThreadBytesDown : kThreadBytesUp) && !known_memory(f))
+        want = (int)std::min<size_t>((bytes + kChunkBytes - 1) / kChunkBytes,
+                                     std::min<size_t>(kCopyThreads, std::thread::hardware_concurrency()));
+    const Borrowed b(c, want, bytes >= kGrowBytes);
     char* dp = static_cast<char*>(d);
     const int T = (int)b.c.size();
     if (T < 2) {
@@ -159,7 +182,7 @@ int copy_fields(mf_ctx* c, void* d, const HostFields& f, bool to_host)
                                                hipMemcpyDeviceToHost, c->stream)
                               : hipMemcpyAsync(dp + v * f.field_bytes, f.fields[v], f.field_bytes,
                                                hipMemcpyHostToDevice, c->stream));
-        MF_HIP(c, hipStreamSynchronize(c->stream));
+        if (to_host) MF_HIP(c, hipStreamSynchronize(c->stream));
         return MF_OK;
     }
     // this thread's own share, and one more thread per further chunk; where
@@ -168,12 +191,13 @@ int copy_fields(mf_ctx* c, void* d, const HostFields& f, bool to_host)
     std::vector<std::thread> th;
     th.reserve(T);
     std::vector<int> mine(1, 0);
+    mine.reserve(T);
     for (int t = 1; t < T; ++t) {
         try {
             th.emplace_back([&, t] {
                 err[t] = copy_chunks(c->device, c->stream, f, dp, bytes, t, T, b.c[t], to_host);
             });
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {  // no thread or no memory for one
             mine.push_back(t);
         }
     }

@@ -1,6 +1,7 @@
 """States and arrays across the transfer paths (pinned in one kernel, pageable,
 several threads through pinned chunks): sizes at the edges of each, odd node
 counts, several host threads at once, and every context closed in between."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -93,3 +94,32 @@ def test_rhs_host_aliased_fields():
     v = u.copy()
     ctx.rhs_host(0.0, v, v)
     assert np.array_equal(v, u)
+
+
+# 40 MiB, from which several threads upload, is 1,310,720 nodes
+@pytest.mark.parametrize("n", [2209, 131072, 262145, 1310719, 1310721])
+def test_pinned_arrays(n):
+    """Arrays that the runtime knows (allocated pinned) cross directly; pageable
+    ones of the same size, and both in one call, give the same."""
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    hip.hipHostFree.argtypes = [C.c_void_p]
+    ctx, u = context(n, n)
+    p = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(p), 4 * 8 * n, 0) == 0
+    try:
+        pin = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), shape=(4 * n,)).reshape(4, n)
+        pin[:] = u
+        ctx.upload(L.MF_BUF_U, pin)
+        assert np.array_equal(ctx.download(L.MF_BUF_U), u)
+        ctx.upload(L.MF_BUF_U, u)
+        pin[:] = 0.0
+        ctx.download(L.MF_BUF_U, pin)
+        assert np.array_equal(pin, u)
+        mixed = [pin[0], np.empty(n), pin[2], np.empty(n)]
+        pin[:] = 0.0
+        fields = (C.POINTER(C.c_double) * 4)(*[m.ctypes.data_as(C.POINTER(C.c_double)) for m in mixed])
+        assert L.lib().mf_state_download(ctx.h, L.MF_BUF_U, fields) == L.MF_OK
+        assert all(np.array_equal(m, v) for m, v in zip(mixed, u))
+    finally:
+        assert hip.hipHostFree(p) == 0
