@@ -236,13 +236,13 @@ int upload_state(mf_ctx* c, double* d_dst, const double* const* fields)
         const Borrowed b(c, 1, true);
         if (!b.c.empty()) {
             copy_part(f, 0, bytes, b.c[0].host, false);
-            if ((rc = launch_soa_to_aos(c, reinterpret_cast<const double*>(b.c[0].host), d_dst))) return rc;
+            if ((rc = launch_soa_to_aos(c, reinterpret_cast<const double*>(b.c[0].host), d_dst, true))) return rc;
             MF_HIP(c, hipStreamSynchronize(c->stream));
             return MF_OK;
         }
     }
     if ((rc = copy_fields(c, c->d_T, f, false))) return rc;
-    return launch_soa_to_aos(c, c->d_T, d_dst);
+    return launch_soa_to_aos(c, c->d_T, d_dst, false);
 }
 
 int download_state(mf_ctx* c, const double* d_src, double* const* fields)
@@ -286,7 +286,7 @@ int rhs_through_pinned(mf_ctx* c, double* d_u, double* d_du, double* const* u, d
     // the input and u's output share a half of the chunk, du has the other
     char *pu = b.c[0].host, *pdu = pu + kDirectBytes;
     copy_part(f, 0, bytes, pu, false);
-    int rc = launch_soa_to_aos(c, reinterpret_cast<const double*>(pu), d_u);
+    int rc = launch_soa_to_aos(c, reinterpret_cast<const double*>(pu), d_u, true);
     if (!rc) rc = run();
     if (!rc) rc = launch_aos_to_soa(c, d_du, reinterpret_cast<double*>(pdu));
     if (!rc) rc = launch_aos_to_soa(c, d_u, reinterpret_cast<double*>(pu));

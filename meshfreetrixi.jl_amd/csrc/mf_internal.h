@@ -341,7 +341,8 @@ int launch_ell_to_rows(mf_ctx* c, const int32_t* d_ell, int32_t* d_rows, int k);
 int launch_ell_to_rows_d(mf_ctx* c, const double* d_ell, double* d_rows, int k);
 int launch_rows_to_ell(mf_ctx* c, const int32_t* d_rows, int32_t* d_ell, int k);
 int launch_rows_to_ell_d(mf_ctx* c, const double* d_rows, double* d_ell, int k);
-int launch_soa_to_aos(mf_ctx* c, const double* d_soa, double* d_aos);
+// host: soa is pinned host memory
+int launch_soa_to_aos(mf_ctx* c, const double* soa, double* d_aos, bool host);
 int launch_aos_to_soa(mf_ctx* c, const double* d_aos, double* d_soa);
 int launch_build_didx(mf_ctx* c);
 // d_group (caller order, may be null): group of each point; the internal
