@@ -229,31 +229,32 @@ __device__ __forceinline__ uint16_t halo_pos(const int32_t* tab, int n, int32_t 
     return (uint16_t)lo;
 }
 
-// The tile's ids (at t cap) and their number (above cap: the halo does not fit).
-__device__ __forceinline__ int halo_finish(int32_t* tab, int T, int cap, const int* cnt, int32_t* ids, int32_t* count,
-                                           int64_t t)
+// The block's tile's ids (at blockIdx.x cap) and their number (above cap: the
+// halo does not fit).
+__device__ __forceinline__ int halo_finish(int32_t* tab, int T, int cap, const int* cnt, int32_t* ids, int32_t* count)
 {
     __syncthreads();
     const int n = *cnt;
-    if (threadIdx.x == 0) count[t] = n;
+    if (threadIdx.x == 0) count[blockIdx.x] = n;
     if (n > cap) return -1;
     halo_sort(tab, T);
-    for (int q = threadIdx.x; q < n; q += kTile) ids[t * cap + q] = tab[q];
+    for (int q = threadIdx.x; q < n; q += kTile) ids[(int64_t)blockIdx.x * cap + q] = tab[q];
     return n;
 }
 
 // Phase A: the union of the tile's stencils, and the tile-major positions of
-// the entries of both stencil copies (0 past the last node).
-__global__ __launch_bounds__(kTile) void k_halo_a(int64_t N, int K, const int32_t* idx, const int32_t* idx_s, int T,
-                                                  int cap, int32_t* ids, int32_t* count, uint16_t* la, uint16_t* la_s)
+// the entries of both stencil copies (0 past the last node).  Tiles t0 on.
+__global__ __launch_bounds__(kTile) void k_halo_a(int64_t t0, int64_t N, int K, const int32_t* idx, const int32_t* idx_s,
+                                                  int T, int cap, int32_t* ids, int32_t* count, uint16_t* la,
+                                                  uint16_t* la_s)
 {
     extern __shared__ int32_t tab[];
     __shared__ int cnt;
-    const int64_t t = blockIdx.x, i = t * kTile + threadIdx.x;
+    const int64_t t = t0 + blockIdx.x, i = t * kTile + threadIdx.x;
     halo_clear(tab, T, &cnt);
     if (i < N)
         for (int s = 0; s < K; ++s) halo_insert(tab, T, cap, &cnt, idx[(int64_t)s * N + i]);
-    const int n = halo_finish(tab, T, cap, &cnt, ids, count, t);
+    const int n = halo_finish(tab, T, cap, &cnt, ids, count);
     if (n < 0) return;
     for (int s = 0; s < K; ++s) {
         const int64_t q = (t * K + s) * kTile + threadIdx.x;
@@ -282,15 +283,15 @@ __global__ __launch_bounds__(kTile) void k_rows_b(int64_t N, const int32_t* deg,
 
 // The union of the rows' entries, and each entry's halo position and source
 // in the slice layout (rows of the global transpose, already in ascending
-// caller index).
-__global__ __launch_bounds__(kTile) void k_halo_b(int64_t N, const int32_t* deg, const int64_t* toff,
+// caller index).  Tiles t0 on.
+__global__ __launch_bounds__(kTile) void k_halo_b(int64_t t0, int64_t N, const int32_t* deg, const int64_t* toff,
                                                   const int32_t* trow, const int64_t* tsrc, const uint8_t* rowb,
                                                   const int64_t* soff, const int32_t* sw, int T, int cap, int32_t* ids,
                                                   int32_t* count, uint16_t* lb, int64_t* src)
 {
     extern __shared__ int32_t tab[];
     __shared__ int cnt;
-    const int64_t t = blockIdx.x;
+    const int64_t t = t0 + blockIdx.x;
     halo_clear(tab, T, &cnt);
     {
         const int64_t i = t * kTile + threadIdx.x;
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(kTile) void k_halo_b(int64_t N, const int32_t* deg,
             for (int e = 0; e < n; ++e) halo_insert(tab, T, cap, &cnt, trow[b + (int64_t)e * kSellC]);
         }
     }
-    const int n = halo_finish(tab, T, cap, &cnt, ids, count, t);
+    const int n = halo_finish(tab, T, cap, &cnt, ids, count);
     if (n < 0) return;
     const int p = threadIdx.x;
     const int64_t i = t * kTile + rowb[t * kTile + p];
@@ -314,11 +315,11 @@ __global__ __launch_bounds__(kTile) void k_halo_b(int64_t N, const int32_t* deg,
     }
 }
 
-// ids[off[t] + q] = tmp[t cap + q]
+// ids[off[t] - off[0] + q] = tmp[t cap + q]
 __global__ void k_halo_pack(const int32_t* tmp, int cap, const int64_t* off, int32_t* ids)
 {
-    const int64_t t = blockIdx.x, o = off[t];
-    const int n = (int)(off[t + 1] - o);
+    const int64_t t = blockIdx.x, o = off[t] - off[0];
+    const int n = (int)(off[t + 1] - off[t]);
     for (int q = threadIdx.x; q < n; q += blockDim.x) ids[o + q] = tmp[t * cap + q];
 }
 
@@ -329,32 +330,75 @@ static int halo_table(int cap)
     return T;
 }
 
-// The halos' sizes (count) to offsets, the packed ids and the largest size;
-// fits = false if some tile's halo has more than cap ids.
-static int pack_halos(mf_ctx* c, int64_t nt, int cap, const int32_t* tmp, const int32_t* count, int64_t** off,
-                      int32_t** ids, int* hmax, int64_t* total, bool* fits)
+// Before its ids are packed a tile has room for cap of them, 3 to 24 times what
+// its halo takes: the tiles go through it in ranges of this size (with room for
+// all of them at once one variable took 96 bytes per node of the cloud).
+constexpr size_t kHaloTempBytes = (size_t)16 << 20;
+
+// The halos by launch(t0, n, ids, count) of the n tiles from t0 on: offsets, the
+// packed ids and the largest size; fits = false if some tile's halo has more
+// than cap ids.
+template <class Launch>
+static int collect_halos(mf_ctx* c, int64_t nt, int cap, Launch launch, int64_t** off, int32_t** ids, int* hmax,
+                         int64_t* total, bool* fits)
 {
-    std::vector<int32_t> n(nt);
-    MF_HIP(c, hipMemcpyAsync(n.data(), count, sizeof(int32_t) * nt, hipMemcpyDeviceToHost, c->stream));
-    MF_HIP(c, hipStreamSynchronize(c->stream));
+    const int64_t range = std::min<int64_t>(nt, (int64_t)(kHaloTempBytes / (sizeof(int32_t) * cap)));
+    int32_t *tmp = nullptr, *count = nullptr;
+    std::vector<int32_t> size(range);
     std::vector<int64_t> o(nt + 1, 0);
+    std::vector<int32_t*> part;  // each range's packed ids
+    part.reserve((size_t)((nt + range - 1) / range));
     *hmax = 0;
-    for (int64_t t = 0; t < nt; ++t) {
-        *hmax = std::max<int>(*hmax, n[t]);
-        o[t + 1] = o[t] + n[t];
-    }
-    *total = o[nt];
-    *fits = *hmax <= cap;
-    if (!*fits) return MF_OK;
-    int rc;
-    if ((rc = upload(c, off, o)) || (rc = dalloc(c, ids, (size_t)o[nt]))) return rc;
-    hipLaunchKernelGGL(k_halo_pack, dim3((unsigned)nt), dim3(kTile), 0, c->stream, tmp, cap, *off, *ids);
-    MF_HIP(c, hipGetLastError());
-    MF_HIP(c, hipStreamSynchronize(c->stream));  // the offsets' host copy ends here
-    return MF_OK;
+    *fits = false;
+    auto body = [&]() -> int {
+        int rc;
+        if ((rc = dalloc(c, &tmp, (size_t)range * cap)) || (rc = dalloc(c, &count, (size_t)range)) ||
+            (rc = dalloc(c, off, (size_t)nt + 1)))
+            return rc;
+        for (int64_t t0 = 0; t0 < nt; t0 += range) {
+            const int64_t n = std::min(range, nt - t0);
+            launch(t0, (unsigned)n, tmp, count);
+            MF_HIP(c, hipGetLastError());
+            MF_HIP(c, hipMemcpyAsync(size.data(), count, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream));
+            MF_HIP(c, hipStreamSynchronize(c->stream));
+            for (int64_t t = 0; t < n; ++t) {
+                *hmax = std::max<int>(*hmax, size[t]);
+                o[t0 + t + 1] = o[t0 + t] + size[t];
+            }
+            if (*hmax > cap) return MF_OK;
+            MF_HIP(c, hipMemcpyAsync(*off + t0, o.data() + t0, sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice,
+                                     c->stream));
+            int32_t* p = nullptr;
+            if ((rc = dalloc(c, &p, (size_t)(o[t0 + n] - o[t0])))) return rc;
+            part.push_back(p);
+            hipLaunchKernelGGL(k_halo_pack, dim3((unsigned)n), dim3(kTile), 0, c->stream, tmp, cap, *off + t0, p);
+            MF_HIP(c, hipGetLastError());
+        }
+        *total = o[nt];
+        if (part.size() == 1) {
+            *ids = part[0];
+            part.clear();
+        } else {
+            if ((rc = dalloc(c, ids, (size_t)o[nt]))) return rc;
+            for (size_t q = 0; q < part.size(); ++q) {
+                const int64_t t0 = (int64_t)q * range, n = std::min(range, nt - t0);
+                MF_HIP(c, hipMemcpyAsync(*ids + o[t0], part[q], sizeof(int32_t) * (o[t0 + n] - o[t0]),
+                                         hipMemcpyDeviceToDevice, c->stream));
+            }
+        }
+        *fits = true;
+        return MF_OK;
+    };
+    int rc = body();
+    const hipError_t e = hipStreamSynchronize(c->stream);  // nothing in flight reads the temporaries
+    if (rc == MF_OK && e != hipSuccess) rc = hip_fail(c, e, "hipStreamSynchronize");
+    dfree(tmp);
+    dfree(count);
+    for (int32_t* p : part) dfree(p);
+    return rc;
 }
 
-static int build_tiles_a(mf_ctx* c, int64_t nt, int32_t** tmp, int32_t** count)
+static int build_tiles_a(mf_ctx* c, int64_t nt)
 {
     const int64_t N = c->N;
     const int K = c->k;
@@ -364,15 +408,14 @@ static int build_tiles_a(mf_ctx* c, int64_t nt, int32_t** tmp, int32_t** count)
     const int T = halo_table(cap);
     const size_t n_la = (size_t)nt * K * kTile;
     int rc;
-    if ((rc = dalloc(c, tmp, (size_t)nt * cap)) || (rc = dalloc(c, count, (size_t)nt)) ||
-        (rc = dalloc(c, &c->d_la, n_la)) || (rc = dalloc(c, &c->d_la_s, n_la)))
-        return rc;
-    hipLaunchKernelGGL(k_halo_a, dim3((unsigned)nt), dim3(kTile), sizeof(int32_t) * T, c->stream, N, K, c->d_idx,
-                       c->d_idx_s, T, cap, *tmp, *count, c->d_la, c->d_la_s);
-    MF_HIP(c, hipGetLastError());
+    if ((rc = dalloc(c, &c->d_la, n_la)) || (rc = dalloc(c, &c->d_la_s, n_la))) return rc;
+    auto launch = [&](int64_t t0, unsigned n, int32_t* ids, int32_t* count) {
+        hipLaunchKernelGGL(k_halo_a, dim3(n), dim3(kTile), sizeof(int32_t) * T, c->stream, t0, N, K, c->d_idx, c->d_idx_s,
+                           T, cap, ids, count, c->d_la, c->d_la_s);
+    };
     bool fits;
     int hmax;
-    if ((rc = pack_halos(c, nt, cap, *tmp, *count, &c->d_ha_off, &c->d_ha_ids, &hmax, &c->ha_total, &fits))) return rc;
+    if ((rc = collect_halos(c, nt, cap, launch, &c->d_ha_off, &c->d_ha_ids, &hmax, &c->ha_total, &fits))) return rc;
     if (!fits) {  // global-memory kernels
         dfree(c->d_la);
         dfree(c->d_la_s);
@@ -385,16 +428,14 @@ static int build_tiles_a(mf_ctx* c, int64_t nt, int32_t** tmp, int32_t** count)
     return MF_OK;
 }
 
-static int build_tiles_b(mf_ctx* c, int64_t nt, int rec_b, int32_t** tmp, int32_t** count)
+static int build_tiles_b(mf_ctx* c, int64_t nt, int rec_b)
 {
     const int64_t N = c->N;
     const int cap = (int)(kTileLdsBytesB / (rec_b * sizeof(double)));
     const int T = halo_table(cap);
     const int64_t nsl = nt * kSlicesPerTile;
     int rc;
-    if ((rc = dalloc(c, tmp, (size_t)nt * cap)) || (rc = dalloc(c, count, (size_t)nt)) ||
-        (rc = dalloc(c, &c->d_rowb, (size_t)nt * kTile)) || (rc = dalloc(c, &c->d_sb_w, (size_t)nsl)))
-        return rc;
+    if ((rc = dalloc(c, &c->d_rowb, (size_t)nt * kTile)) || (rc = dalloc(c, &c->d_sb_w, (size_t)nsl))) return rc;
     hipLaunchKernelGGL(k_rows_b, dim3((unsigned)nt), dim3(kTile), 0, c->stream, N, c->d_tdeg, c->d_rowb, c->d_sb_w);
     MF_HIP(c, hipGetLastError());
     std::vector<int32_t> sw(nsl);
@@ -406,13 +447,14 @@ static int build_tiles_b(mf_ctx* c, int64_t nt, int rec_b, int32_t** tmp, int32_
     if ((rc = upload(c, &c->d_sb_off, soff)) || (rc = dalloc(c, &c->d_lb, (size_t)ne)) ||
         (rc = dalloc(c, &c->d_tb_src, (size_t)ne)))
         return rc;
-    hipLaunchKernelGGL(k_halo_b, dim3((unsigned)nt), dim3(kTile), sizeof(int32_t) * T, c->stream, N, c->d_tdeg,
-                       c->d_sell_off, c->d_trow, c->d_tsrc, c->d_rowb, c->d_sb_off, c->d_sb_w, T, cap, *tmp, *count,
-                       c->d_lb, c->d_tb_src);
-    MF_HIP(c, hipGetLastError());
+    auto launch = [&](int64_t t0, unsigned n, int32_t* ids, int32_t* count) {
+        hipLaunchKernelGGL(k_halo_b, dim3(n), dim3(kTile), sizeof(int32_t) * T, c->stream, t0, N, c->d_tdeg, c->d_sell_off,
+                           c->d_trow, c->d_tsrc, c->d_rowb, c->d_sb_off, c->d_sb_w, T, cap, ids, count, c->d_lb,
+                           c->d_tb_src);
+    };
     bool fits;
     int hmax;
-    if ((rc = pack_halos(c, nt, cap, *tmp, *count, &c->d_hb_off, &c->d_hb_ids, &hmax, &c->hb_total, &fits))) return rc;
+    if ((rc = collect_halos(c, nt, cap, launch, &c->d_hb_off, &c->d_hb_ids, &hmax, &c->hb_total, &fits))) return rc;
     if (!fits) return MF_OK;  // global-memory transposed gather
     if ((rc = dalloc(c, &c->d_twb, (size_t)ne)) || (rc = dalloc(c, &c->d_twb32, (size_t)ne))) return rc;
     hipLaunchKernelGGL(k_fill_tile_weights, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, c->stream, ne,
@@ -431,15 +473,10 @@ static int build_tiles_b(mf_ctx* c, int64_t nt, int rec_b, int32_t** tmp, int32_
 int build_tiles(mf_ctx* c, bool want_b, int rec_b)
 {
     const int64_t nt = (c->N + kTile - 1) / kTile;
-    int rc = MF_OK;
-    int32_t *tmp = nullptr, *count = nullptr;
     if (!c->tried_a) {
         free_tiles(c);
         c->tried_a = true;
-        rc = build_tiles_a(c, nt, &tmp, &count);
-        if (rc) (void)hipStreamSynchronize(c->stream);  // nothing in flight reads them
-        dfree(tmp);
-        dfree(count);
+        const int rc = build_tiles_a(c, nt);
         if (rc) return rc;
     }
     if (!want_b || !c->tiles_a || c->tried_b) return MF_OK;
@@ -447,12 +484,7 @@ int build_tiles(mf_ctx* c, bool want_b, int rec_b)
     free_tiles_b(c);
     c->tried_b = true;
     c->tiles_b_rec = rec_b;
-    tmp = count = nullptr;
-    rc = build_tiles_b(c, nt, rec_b, &tmp, &count);
-    if (rc) (void)hipStreamSynchronize(c->stream);
-    dfree(tmp);
-    dfree(count);
-    return rc;
+    return build_tiles_b(c, nt, rec_b);
 }
 
 }  // namespace mf

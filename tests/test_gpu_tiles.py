@@ -188,3 +188,29 @@ def test_transposed_halos_that_do_not_fit():
             assert (ctx.tile_info()["tiles_a"], ctx.tile_info()["tiles_b"]) == (tiles, 0)
             out.append(du)
         assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
+
+
+def test_halos_in_ranges():
+    """One variable and more tiles than one range of the temporary ids holds (682
+    for the stencils, 512 for the transposed entries)."""
+    rng = np.random.default_rng(12)
+    n = 682 * 256 + 4001
+    ctx = L.Context(0)
+    ctx.set_equations(L.MF_EQ_ADVECTION_2D, 1.0, 0.5)
+    ctx.set_points(rng.random(n), rng.random(n))
+    idx = ctx.knn(5)[0]
+    operators(ctx, idx, rng)
+    u, lam = rng.standard_normal((1, n)), rng.standard_normal((1, n))
+    out = []
+    for tiles in (0, 1):
+        ctx.set_tuning(L.MF_TUNE_TILES, tiles)
+        ctx.upload(L.MF_BUF_U, u)
+        ctx.upload(L.MF_BUF_AUX0, lam)
+        ctx.rhs_vjp(0.0)
+        ctx.rhs(0.0)
+        out.append((ctx.download(L.MF_BUF_AUX1), ctx.download(L.MF_BUF_DU)))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    ti = ctx.tile_info()
+    assert ti["tiles_a"] and ti["tiles_b"]
+    assert (ti["halo_a_total"], ti["halo_b_total"], ti["halo_a_max"], ti["halo_b_max"],
+            ti["b_entries_padded"]) == expected(idx, ctx.node_order())
