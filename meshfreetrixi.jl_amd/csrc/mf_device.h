@@ -268,23 +268,6 @@ __device__ __forceinline__ void mean_from_partials(const double* psum, int npart
     for (int v = 0; v < 4; ++v) mean[v] = acc[v] / (double)(4 * N);
 }
 
-// ninf from the per-block partial lexicographic maxima, zeros -> eps().
-__device__ __forceinline__ void ninf_from_partials(const double* pmax, int nparts, double* ninf)
-{
-    double best[4] = {-1.0, -1.0, -1.0, -1.0};
-    for (int b = threadIdx.x; b < nparts; b += kBlock) {
-        double c[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) c[v] = pmax[4 * b + v];
-        if (lex_less(best, c))
-#pragma unroll
-            for (int v = 0; v < 4; ++v) best[v] = c[v];
-    }
-    block_lexmax4(best);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) ninf[v] = (best[v] == 0.0) ? DBL_EPSILON : best[v];
-}
-
 // XCD-aware logical block (the remap of remapped_node).
 __device__ __forceinline__ int64_t remapped_block()
 {
