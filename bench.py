@@ -123,7 +123,9 @@ def measured_traffic(kernel, tuning, side, tiled, mode="f64_ref"):
         family, tail = "k_rhs_transpose<4, %d," % tm, "%s, 1>(mf::RhsArgs)" % tl
     else:
         kern = "k_rhs_ref" if mode == "f64_ref" else "k_rhs_f64"
-        want = "%s<4, 30, 0, true, %d, %s>" % (kern, tuning[mode]["flux"] or 5, tl)
+        # entries per batch and whether two batches are in flight in turn
+        bt, two = {3: (3, "false"), 6: (3, "true"), 10: (5, "true")}.get(tuning[mode]["flux"], (5, "false"))
+        want = "%s<4, 30, 0, true, %d, %s, %s>" % (kern, bt, two if tiled else "false", tl)
         family, tail = "%s<4, 30, 0, true," % kern, "%s>(mf::RhsArgs)" % tl
     names = [n for n in tab["kernels"] if want in n] or \
         [n for n in tab["kernels"] if family in n and n.endswith(tail)]
@@ -520,14 +522,14 @@ def weights_cpu(x, y, ptr, ridx, gpu_w, sample):
 PROFILE_COMMANDS = {
     "traffic": [
         "cd /tmp && export TMPDIR=/tmp && timeout -s KILL 200 rocprofv3 --pmc FETCH_SIZE --output-format csv "
-        "-d $REPO/gpurun_out/prof_fetch -o fetch -- python3 $REPO/bench.py --steps 10 --warmup 2 --no-extras --no-cpu",
+        "-d $REPO/gpurun_out/prof_fetch -o fetch -- python3 $REPO/bench.py --profile-run --steps 5",
         "cd /tmp && export TMPDIR=/tmp && timeout -s KILL 200 rocprofv3 --pmc WRITE_SIZE --output-format csv "
-        "-d $REPO/gpurun_out/prof_write -o write -- python3 $REPO/bench.py --steps 10 --warmup 2 --no-extras --no-cpu",
+        "-d $REPO/gpurun_out/prof_write -o write -- python3 $REPO/bench.py --profile-run --steps 5",
         "python3 bench.py --profile-summary traffic gpurun_out/prof_fetch gpurun_out/prof_write",
     ],
     "trace": [
         "cd /tmp && export TMPDIR=/tmp && timeout -k 10 300 rocprofv3 --kernel-trace --stats --output-format csv "
-        "-d $REPO/gpurun_out/prof_trace -o trace -- python3 $REPO/bench.py --steps 200 --warmup 10 --headline-only",
+        "-d $REPO/gpurun_out/prof_trace -o trace -- python3 $REPO/bench.py --profile-run --steps 30",
         "python3 bench.py --profile-summary trace gpurun_out/prof_trace",
     ],
     "weights": [
@@ -634,9 +636,9 @@ def profile_summary(kind, dirs):
         lines, _ = _trace_table(dirs[0])
         text = ("# Kernel trace: Euler + residual viscosity rhs!, 262,144 nodes, k = 30\n\n"
                 "Commands (from the repository root, on one MI355X):\n\n```\n%s\n```\n\n"
-                "Top kernels by total time.  The run includes the autotuner's sweep (every load-batch variant "
-                "of each precision inside whole rhs! calls) and the headline (reference-order FP64) timing "
-                "loop, so each kernel's average is over whole-rhs! sequences.\n\n%s\n" % (cmds, "\n".join(lines)))
+                "Top kernels by total time.  The run calls rhs! eagerly, 30 times with every load-batch variant "
+                "of each precision (the transposed kernel's batches in turn), so each kernel's average is over "
+                "whole-rhs! sequences.\n\n%s\n" % (cmds, "\n".join(lines)))
     else:  # weights
         lines, rows = _trace_table(dirs[0], top=8)
         cnt = _counter_medians(dirs[1])
@@ -670,6 +672,9 @@ def main():
     ap.add_argument("--no-extras", action="store_true", help="skip adjoint and batched weights")
     ap.add_argument("--headline-only", action="store_true",
                     help="time the headline mode's rhs! only and print its figures (for profiled runs)")
+    ap.add_argument("--profile-run", action="store_true",
+                    help="only the calibration copies and --steps eager rhs! calls with every load-batch variant "
+                         "of each precision (for profiled runs: no graphs, no timing)")
     ap.add_argument("--weights-only", action="store_true",
                     help="time only the batched weights (1,048,576 ragged stencils) and print their JSON")
     ap.add_argument("--profile-summary", nargs="+", metavar=("KIND", "DIR"),
@@ -716,6 +721,14 @@ def main():
     # three SSPRK33 steps with the history callback so the residual viscosity is live
     ctx.ssprk33(0.0, info["dt"], 3, flags=L.MF_STEP_HISTORY)
     t_now = 3 * info["dt"]
+    if args.profile_run:
+        for prec in (L.MF_PREC_F64_REF, L.MF_PREC_F64, L.MF_PREC_SPLIT32):
+            for q, f in enumerate(tune.FLUX_BATCHES[k]):
+                ctx.set_tuning(L.MF_TUNE_FLUX_BATCH, f, prec)
+                ctx.set_tuning(L.MF_TUNE_TRANSPOSE_BATCH, tune.TRANSPOSE_BATCHES[q % 3], prec)
+                for _ in range(args.steps):
+                    ctx.rhs(t_now, prec)
+        return
     log("knn %.1f ms, weights %.1f ms; warmup %d rhs!" % (1e3 * info["t_knn"], 1e3 * info["t_weights"],
                                                           args.warmup))
     ctx.time_rhs(t_now, L.MF_PREC_F64_REF, max(1, args.warmup))

@@ -1353,9 +1353,10 @@ static bool stage_handover(const mf_ctx* c, bool limiter)
 // T's and U's at this step's stage times t + dt/2 and t + dt, S's at the
 // next step's t_next + dt.  With raw_s the stored S has had neither (the
 // boundary conditions changed since it was written, or the call that wrote it
-// did not hand over): its rhs! runs the pass and the sums itself.  The time moves on in the stage kernels: the
-// second stage writes t_next = t + dt, the last makes it t (with the history
-// callback, which needs both, the callback does).
+// did not hand over): its rhs! runs the pass and the sums itself.  The time
+// moves on in the stage kernels: the second stage writes t_next = t + dt, the
+// last makes it t (with the history callback, which needs both, the callback
+// does).
 static int ssprk_step(mf_ctx* c, double dt, int prec, bool limiter, bool history, bool hand, bool raw_s = false)
 {
     int rc;
