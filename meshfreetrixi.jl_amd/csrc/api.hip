@@ -535,15 +535,12 @@ int mf_set_stencil(mf_ctx* c, const int32_t* idx, int64_t n_points, int k)
     if ((rc = set_k(c, k))) return rc;
     int32_t* rows = nullptr;
     if ((rc = dalloc(c, &rows, (size_t)k * c->N))) return rc;
-    if ((rc = copy_array(c, rows, idx, sizeof(int32_t) * k * c->N, false))) {
-        dfree(rows);
-        return rc;
-    }
-    if ((rc = launch_rows_to_ell(c, rows, c->d_idx, k))) return rc;
-    if ((rc = stencil_ready(c))) return rc;
-    MF_HIP(c, hipStreamSynchronize(c->stream));
+    rc = copy_array(c, rows, idx, sizeof(int32_t) * k * c->N, false);
+    if (!rc) rc = launch_rows_to_ell(c, rows, c->d_idx, k);
+    if (!rc) rc = stencil_ready(c);
+    const hipError_t e = hipStreamSynchronize(c->stream);  // also after an error: the copy reads idx no more
     dfree(rows);
-    return MF_OK;
+    return rc ? rc : e != hipSuccess ? hip_fail(c, e, "hipStreamSynchronize") : MF_OK;
 }
 
 static int alloc_op(mf_ctx* c, int target)
@@ -1239,7 +1236,10 @@ int mf_rhs_host(mf_ctx* c, double t, int precision, double* const* u, double* co
         if (rc || done) return rc;
     }
     if ((rc = upload_fields(c, c->d_buf[MF_BUF_U], u))) return rc;
-    if ((rc = mf_rhs(c, t, precision))) return rc;
+    if ((rc = mf_rhs(c, t, precision))) {
+        (void)hipStreamSynchronize(c->stream);  // the upload reads the caller's arrays no more
+        return rc;
+    }
     if ((rc = download_fields(c, c->d_buf[MF_BUF_DU], du))) return rc;
     return download_fields(c, c->d_buf[MF_BUF_U], u);
 }

@@ -241,8 +241,10 @@ int upload_state(mf_ctx* c, double* d_dst, const double* const* fields)
             return MF_OK;
         }
     }
-    if ((rc = copy_fields(c, c->d_T, f, false))) return rc;
-    return launch_soa_to_aos(c, c->d_T, d_dst, false);
+    rc = copy_fields(c, c->d_T, f, false);
+    if (!rc) rc = launch_soa_to_aos(c, c->d_T, d_dst, false);
+    if (rc) (void)hipStreamSynchronize(c->stream);  // the caller's arrays are read no more
+    return rc;
 }
 
 int download_state(mf_ctx* c, const double* d_src, double* const* fields)

@@ -123,3 +123,26 @@ def test_pinned_arrays(n):
         assert all(np.array_equal(m, v) for m, v in zip(mixed, u))
     finally:
         assert hip.hipHostFree(p) == 0
+
+
+@pytest.mark.parametrize("n", [262145, 1310719])
+def test_refused_call_reads_no_more(n):
+    """A refused rhs! has taken its pinned arrays when it returns: writing to
+    them at once changes nothing of the state that it uploaded."""
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    hip.hipHostFree.argtypes = [C.c_void_p]
+    ctx, u = context(n, n)
+    p = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(p), 4 * 8 * n, 0) == 0
+    try:
+        pin = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), shape=(4 * n,)).reshape(4, n)
+        pin[:] = u
+        du = np.empty((4, n))
+        rc = L.lib().mf_rhs_host(ctx.h, 0.0, L.MF_PREC_F64, ctx._fields(pin), ctx._fields(du))
+        pin[::-1] = -1.0
+        assert rc == L.MF_ERR_STATE  # no operator
+        assert np.array_equal(ctx.download(L.MF_BUF_U), u)
+    finally:
+        ctx.close()
+        assert hip.hipHostFree(p) == 0
